@@ -207,11 +207,15 @@ struct Attn {
 };
 size_t attention_ws_bytes(const Attn &a);
 void attention(hipStream_t s, const Attn &a, float *ws);
-// Reference-order prefill (exact, seq_q > 4, head_dim 64 or 128) on the fp32
-// matrix cores (attn_exact.hip).
+// Reference-order attention on the fp32 matrix cores takes the call: head_dim
+// a multiple of 8 up to 128, rows it can copy 16 bytes at a time, and decode
+// scores of one (batch, head) within its workspace cap (attn_exact.hip).
+bool attention_exact_supported(const Attn &a);
+// Whether it runs as decode (up to 4 query rows, and some calls of a few more).
+bool attention_exact_decodes(const Attn &a);
+// Reference-order prefill.
 void attention_exact_prefill(hipStream_t s, const Attn &a);
-// Reference-order decode (exact, seq_q <= 4, head_dim 64 or 128): scores,
-// then the output chain (attn_exact.hip); ws holds
+// Reference-order decode: scores, then the output chain; ws holds
 // attention_exact_decode_ws_bytes(a).
 size_t attention_exact_decode_ws_bytes(const Attn &a);
 void attention_exact_decode(hipStream_t s, const Attn &a, float *ws);

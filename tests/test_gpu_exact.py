@@ -232,6 +232,31 @@ def test_attention_reference_order_prefill_shapes(exact_gpu, b, h, sq, sk, d, ca
     assert bits(got, block_oracle.attention_threaded(Q, K, V, causal, mask=M, avx2=True))
 
 
+@pytest.mark.parametrize("d", [8, 32, 40, 56, 80, 88, 96, 120])
+@pytest.mark.parametrize("b,h,sq,sk,causal,mask", [
+    (2, 2, 1, 129, 1, None), (1, 3, 4, 300, 0, "normal"),      # decode: one tile per scores wave, ragged keys
+    (1, 2, 6, 1100, 1, None),                                  # a few rows behind a long context
+    (1, 2, 33, 65, 1, "row"), (2, 1, 70, 20, 1, None),         # rows shared by the waves of a workgroup
+    (1, 1, 31, 64, 0, "inf"),
+    (8, 33, 130, 64, 1, None)])                                # 128 rows per workgroup (the grid fills the chip)
+def test_attention_reference_order_head_sizes(exact_gpu, b, h, sq, sk, d, causal, mask):
+    """Head sizes that fill no tile, on each kernel of the reference order, bit for bit."""
+    if b * h > 100 and d not in (40, 80, 120):
+        pytest.skip("the large grid runs on three of the head sizes")
+    Q = RNG.standard_normal((b, h, sq, d)).astype(np.float32)
+    K = RNG.standard_normal((b, h, sk, d)).astype(np.float32)
+    V = RNG.standard_normal((b, h, sk, d)).astype(np.float32)
+    M = None
+    if mask:
+        M = RNG.standard_normal((b, h, sq, sk)).astype(np.float32)
+        if mask == "inf":
+            M[..., : sk // 3] = -np.inf
+        if mask == "row":
+            M[0, 0, 3, :] = -np.inf
+    got = g.attention(exact_gpu, Q, K, V, M, causal)
+    assert bits(got, block_oracle.attention_threaded(Q, K, V, causal, mask=M, avx2=True))
+
+
 def test_attention_reference_order_nonfinite_v_masked(exact_gpu):
     """Infinite and NaN values of V at keys some rows never weigh: the matrix
     core would turn v * 0 into NaN where the reference skips the key, so
