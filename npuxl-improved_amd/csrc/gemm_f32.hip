@@ -1495,7 +1495,7 @@ size_t gemm_f32_ws_bytes(const F32Gemm &p)
     return splits > 1 ? static_cast<size_t>(splits) * p.M * p.N * sizeof(float) : 0;
 }
 
-static void splitk_reduce(hipStream_t s, const F32Gemm &p, const float *ws, uint32_t splits)
+void splitk_reduce(hipStream_t s, const F32Gemm &p, const float *ws, uint32_t splits)
 {
     const uint64_t total = static_cast<uint64_t>(p.M) * p.N;
     gemm_f32_splitk_reduce<<<dim3(static_cast<uint32_t>((total + kThreads - 1) / kThreads)), kThreads, 0, s>>>(

@@ -145,6 +145,13 @@ void gemm_f32(hipStream_t s, const F32Gemm &p, float *ws);
 size_t gemv_f32_ws_bytes(const F32Gemm &p);
 bool gemv_f32_supported(const F32Gemm &p);
 void gemv_f32(hipStream_t s, const F32Gemm &p, float *ws);
+// Few rows (skinny_f32.hip): M <= 64, op(A) = A, no cull and no requested K
+// depth, where it is the faster one; ws holds skinny_f32_ws_bytes(p).
+bool skinny_f32_takes(const F32Gemm &p);
+size_t skinny_f32_ws_bytes(const F32Gemm &p);
+void skinny_f32(hipStream_t s, const F32Gemm &p, float *ws);
+// C = epilogue of the sum over z of ws[z][m][n], z ascending (gemm_f32.hip).
+void splitk_reduce(hipStream_t s, const F32Gemm &p, const float *ws, uint32_t splits);
 
 // ---- transformer ops (ops.hip) ----
 void rmsnorm(hipStream_t s, const float *X, const float *W, float *Y, uint32_t rows,

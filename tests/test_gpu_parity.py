@@ -589,6 +589,42 @@ def test_matmul_f32_strided_operands(gpu, M, K, N, ta, tb):
     assert rel(got, want) <= 1e-4
 
 
+@pytest.mark.parametrize("M,K,N,tb,lda_pad,ldb_pad", [
+    # lanes along K ([N][K], M <= 8, from 8M weights): N % 4 rows left over, one
+    # to sixteen waves a row group, a last block of 256 depths that is not whole,
+    # activations staged in two chunks
+    (1, 8192, 1025, 1, 0, 0), (3, 2052, 4099, 1, 4, 8), (8, 8448, 1000, 1, 0, 0), (5, 4100, 9002, 1, 0, 4),
+    # the matrix core, [N][K]: one depth, a depth past a chunk, 16 / 17 / 64 rows, unaligned rows
+    (1, 1, 1, 1, 0, 0), (16, 1028, 33, 1, 0, 0), (17, 2052, 70, 1, 0, 4), (64, 500, 129, 1, 0, 0), (9, 333, 65, 1, 1, 3),
+    # [K][N]: 64, 32 and 16 columns a workgroup, with K split and not, widths left over
+    (4, 3000, 132, 0, 0, 0), (16, 4100, 68, 0, 4, 4), (33, 1999, 200, 0, 1, 0), (64, 2048, 4, 0, 0, 0),
+    (8, 2048, 70, 0, 0, 2), (31, 4097, 34, 0, 0, 0), (12, 1500, 1503, 0, 0, 2), (64, 1030, 17, 0, 0, 0),
+    (2, 513, 1000, 0, 0, 0), (32, 15, 7, 0, 0, 0)])
+def test_matmul_f32_few_rows(gpu, M, K, N, tb, lda_pad, ldb_pad):
+    """Few rows (skinny_f32.hip) at the edges of its tiles and rules.  Every
+    product and sum is f32, in chains of at most K / 16 terms: the error is
+    near sqrt(K / 16) 2^-24 of the largest term, below 1e-5 of the result."""
+    rng = np.random.default_rng(M + 7 * K + 13 * N)
+    lda, ldb = K + lda_pad, (K if tb else N) + ldb_pad
+    A = rng.standard_normal((M, lda)).astype(np.float32)
+    B = rng.standard_normal((N if tb else K, ldb)).astype(np.float32)
+    A[:, K:] = np.nan                                   # padding is not read into a result
+    B[:, (K if tb else N):] = np.nan
+    bias = rng.standard_normal(N).astype(np.float32)
+    C0 = rng.standard_normal((M, N)).astype(np.float32)
+    ba, bb, bbias, bc = gpu.upload(A), gpu.upload(B), gpu.upload(bias), gpu.upload(C0)
+    try:
+        gpu.run(abi.OP_MATMUL_F32, A=ba, B=bb, bias=bbias.ptr, C=bc, M=M, K=K, N=N, lda=lda, ldb=ldb, trans_b=tb,
+                alpha=1.5, beta=0.5, epilogue=abi.EPI_RELU)
+        got = gpu.download(bc, np.float32, (M, N))
+    finally:
+        for b in (ba, bb, bbias, bc):
+            gpu.free(b)
+    want = oracle.matmul_f32(np.ascontiguousarray(A[:, :K]), np.ascontiguousarray(B[:, :K if tb else N]), C0, bias,
+                             M, K, N, 0, tb, 1.5, 0.5, abi.EPI_RELU, acc64=True)
+    assert rel(got, want) <= 1e-5
+
+
 @pytest.mark.parametrize("M,K,N,pad", [(1, 4096, 32000, 0), (4, 1000, 25600, 0), (8, 300, 25602, 0),
                                        (3, 17, 26000, 6), (5, 1, 25600, 0), (2, 2000, 25601, 0),
                                        (7, 513, 25800, 3), (6, 4100, 25472, 0), (1, 12000, 25600, 0),
