@@ -68,9 +68,12 @@ __device__ __forceinline__ void store_out(const F32Gemm &p, uint32_t m, uint32_t
     *dst = dev::epilogue(out, p.epilogue);
 }
 
-// MG groups of 16 rows, CB blocks of 16 columns, NT: B stored [N][K], VA and
-// VB: floats per load of A and of B (B stored [K][N]: VB = CB).
-template <int MG, int CB, bool NT, int VA, int VB, int W, int U>
+// MG groups of 16 rows (from row 16 MG blockIdx.z on), CB blocks of 16 columns,
+// NT: B stored [N][K].  Loads of four floats need no more than 4-byte
+// alignment.  The last K % 4 depths, which a vector would run past (what
+// follows them may be NaN), are one step of their own; a vector that runs past
+// N only feeds columns that are not stored.
+template <int MG, int CB, bool NT, int W, int U>
 __global__ __launch_bounds__(64 * W) void skinny_f32_kernel(F32Gemm p, uint32_t k_per_split, float *ws)
 {
     extern __shared__ float red[];   // [W][16 MG][16 CB]
@@ -79,10 +82,12 @@ __global__ __launch_bounds__(64 * W) void skinny_f32_kernel(F32Gemm p, uint32_t 
     const int g = lane >> 4, c = lane & 15;
     const uint32_t n0 = blockIdx.x * (16 * CB);
 
-    const auto ra = buffer(p.A, (static_cast<uint64_t>(p.M - 1) * p.lda + p.K) * 4);
+    const uint32_t K4 = p.K & ~3u;
+    const uint32_t m0 = blockIdx.z * (16 * MG), mrows = min(16u * MG, p.M - m0);
+    const auto ra = buffer(p.A + static_cast<uint64_t>(m0) * p.lda, (static_cast<uint64_t>(mrows - 1) * p.lda + p.K) * 4);
     uint32_t arow[MG], brow[CB];
 #pragma unroll
-    for (int m = 0; m < MG; ++m) arow[m] = min(16u * m + c, p.M - 1) * p.lda;   // rows past M are not stored
+    for (int m = 0; m < MG; ++m) arow[m] = min(16u * m + c, mrows - 1) * p.lda;   // rows past M are not stored
     if constexpr (NT) {
 #pragma unroll
         for (int b = 0; b < CB; ++b) brow[b] = min(16u * b + c, p.N - 1 - n0) * p.ldb;
@@ -97,28 +102,23 @@ __global__ __launch_bounds__(64 * W) void skinny_f32_kernel(F32Gemm p, uint32_t 
         float b[U][NT ? CB : 4][NT ? 4 : CB];
     };
     auto fetch = [&](Chunk &t, uint32_t kc) {
-        const auto rn = buffer(p.B + static_cast<uint64_t>(min(kc, p.K - 1)) * p.ldb + n0,
-                               kc < p.K ? (static_cast<uint64_t>(p.K - kc - 1) * p.ldb + (p.N - n0)) * 4 : 0);
+        const auto rn = buffer(p.B + static_cast<uint64_t>(kc < K4 ? kc : 0) * p.ldb + n0,
+                               kc < K4 ? (static_cast<uint64_t>(K4 - kc - 1) * p.ldb + (p.N - n0)) * 4 : 0);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const uint32_t k = kc + 16 * u + 4 * g;
             if constexpr (NT) {
 #pragma unroll
                 for (int b = 0; b < CB; ++b)
-#pragma unroll
-                    for (int s = 0; s < 4; s += VB)
-                        load<VB, kNontemporal>(rt, k + s < p.K ? (brow[b] + k + s) * 4 : kOut, &t.b[u][b][s]);
+                    load<4, kNontemporal>(rt, k < K4 ? (brow[b] + k) * 4 : kOut, t.b[u][b]);
             } else {
-                // rows past K lie past the buffer's end
+                // rows past K4 lie past the buffer's end
 #pragma unroll
                 for (int s = 0; s < 4; ++s)
                     load<CB, kNontemporal>(rn, ncol + (16 * u + 4 * g + s) * p.ldb * 4, t.b[u][s]);
             }
 #pragma unroll
-            for (int m = 0; m < MG; ++m)
-#pragma unroll
-                for (int s = 0; s < 4; s += VA)
-                    load<VA, 0>(ra, k + s < p.K ? (arow[m] + k + s) * 4 : kOut, &t.a[u][m][s]);
+            for (int m = 0; m < MG; ++m) load<4, 0>(ra, k < K4 ? (arow[m] + k) * 4 : kOut, t.a[u][m]);
         }
     };
     f32x4 acc[MG][CB];
@@ -138,17 +138,36 @@ __global__ __launch_bounds__(64 * W) void skinny_f32_kernel(F32Gemm p, uint32_t 
                         acc[m][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(t.a[u][m][s], NT ? t.b[u][b][s] : t.b[u][s][b],
                                                                          acc[m][b], 0, 0, 0);
     };
-    const uint32_t kb = blockIdx.y * k_per_split, ke = min(p.K, kb + k_per_split);
+    const uint32_t kb = blockIdx.y * k_per_split, ke = min(K4, kb + k_per_split);
     constexpr uint32_t step = 16 * U * W;
     Chunk x, y;
     uint32_t kc = kb + 16 * U * wave;
     if (kc < ke) fetch(x, kc);
     for (; kc < ke; kc += 2 * step) {
-        fetch(y, kc + step < ke ? kc + step : p.K);
+        fetch(y, kc + step < ke ? kc + step : K4);
         multiply(x);
         if (kc + step >= ke) break;
-        fetch(x, kc + 2 * step < ke ? kc + 2 * step : p.K);
+        fetch(x, kc + 2 * step < ke ? kc + 2 * step : K4);
         multiply(y);
+    }
+
+    if (K4 < p.K && blockIdx.y + 1 == gridDim.y && wave == W - 1) {   // uniform
+        const uint32_t k = K4 + g;
+        const auto rl = buffer(p.B + static_cast<uint64_t>(K4) * p.ldb + n0,
+                               NT ? 0 : (static_cast<uint64_t>(p.K - 1 - K4) * p.ldb + (p.N - n0)) * 4);
+        float a[MG], b[CB];
+#pragma unroll
+        for (int m = 0; m < MG; ++m) load<1, 0>(ra, k < p.K ? (arow[m] + k) * 4 : kOut, &a[m]);
+        if constexpr (NT) {
+#pragma unroll
+            for (int i = 0; i < CB; ++i) load<1, 0>(rt, k < p.K ? (brow[i] + k) * 4 : kOut, &b[i]);
+        } else {
+            load<CB, 0>(rl, k < p.K ? ncol + g * p.ldb * 4 : kOut, b);
+        }
+#pragma unroll
+        for (int i = 0; i < CB; ++i)
+#pragma unroll
+            for (int m = 0; m < MG; ++m) acc[m][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m], b[i], acc[m][i], 0, 0, 0);
     }
 
     // acc[m][b][i]: row 16m + 4g + i, column 16b + c ([N][K]) or CB c + b.
@@ -161,7 +180,7 @@ __global__ __launch_bounds__(64 * W) void skinny_f32_kernel(F32Gemm p, uint32_t 
                 red[(wave * 16 * MG + 16 * m + 4 * g + i) * 16 * CB + (NT ? 16 * b + c : CB * c + b)] = acc[m][b][i];
     __syncthreads();
     for (uint32_t o = tid; o < 16 * MG * 16 * CB; o += 64 * W) {
-        const uint32_t m = o / (16 * CB), n = n0 + o % (16 * CB);
+        const uint32_t m = m0 + o / (16 * CB), n = n0 + o % (16 * CB);
         if (m >= p.M || n >= p.N) continue;
         float v = 0.0f;
 #pragma unroll
@@ -178,7 +197,7 @@ struct Plan {
     uint32_t splits = 1, k_per = 0;
 };
 
-template <int MG, int CB, bool NT, int VA, int VB, int W, int U>
+template <int MG, int CB, bool NT, int W, int U>
 void launch(hipStream_t s, const F32Gemm &p, const Plan &x, float *ws)
 {
     constexpr size_t lds = static_cast<size_t>(W) * 16 * MG * 16 * CB * sizeof(float);
@@ -186,32 +205,21 @@ void launch(hipStream_t s, const F32Gemm &p, const Plan &x, float *ws)
     if constexpr (lds > 65536) {
         static std::atomic<bool> optin{false};   // launches may come from several host threads
         if (!optin)
-            optin = hipFuncSetAttribute(reinterpret_cast<const void *>(skinny_f32_kernel<MG, CB, NT, VA, VB, W, U>),
+            optin = hipFuncSetAttribute(reinterpret_cast<const void *>(skinny_f32_kernel<MG, CB, NT, W, U>),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) == hipSuccess;
     }
-    skinny_f32_kernel<MG, CB, NT, VA, VB, W, U><<<dim3((p.N + 16 * CB - 1) / (16 * CB), x.splits), 64 * W, lds, s>>>(
-        p, x.k_per, x.splits > 1 ? ws : nullptr);
+    const dim3 grid((p.N + 16 * CB - 1) / (16 * CB), x.splits, (p.M + 16 * MG - 1) / (16 * MG));
+    skinny_f32_kernel<MG, CB, NT, W, U><<<grid, 64 * W, lds, s>>>(p, x.k_per, x.splits > 1 ? ws : nullptr);
 }
 
 // Sixteen waves a workgroup where their registers allow it (128 a lane), and
 // as many depths in flight as eight waves' 256 hold.
-template <int MG, bool NT, int VA, int VB>
+template <int MG, bool NT>
 void launch_matrix(hipStream_t s, const F32Gemm &p, const Plan &x, float *ws)
 {
-    if constexpr (NT) {
-        if constexpr (MG == 1) {
-            if (x.cb == 1) {
-                launch<1, 1, true, VA, VB, 16, 4>(s, p, x, ws);
-                return;
-            }
-        }
-        launch<MG, 4, true, VA, VB, 8, 2>(s, p, x, ws);
-    } else if constexpr (VB == 4) {
-        launch<MG, 4, false, VA, 4, 8, 2>(s, p, x, ws);
-    } else {
-        constexpr bool wide = MG * VB <= 2;
-        launch<MG, VB, false, VA, VB, wide ? 16 : 8, MG * VB <= 4 ? 4 : 2>(s, p, x, ws);
-    }
+    if (x.cb == 4) launch<MG, 4, NT, 8, 2>(s, p, x, ws);
+    else if (x.cb == 2) launch<MG, 2, NT, 8, 4>(s, p, x, ws);
+    else launch<MG, 1, NT, MG <= 2 ? 16 : 8, 4>(s, p, x, ws);
 }
 
 // ---------------------------------------------------------------------------
@@ -260,6 +268,7 @@ __global__ __launch_bounds__(64 * NTW) void gemv_f32_nt_kernel(F32Gemm p, uint32
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t per_wg = NTW / waves_per, slot = wave / waves_per, share = wave % waves_per;
     const uint32_t groups = (p.N + NTR - 1) / NTR, step = 256 * waves_per;
+    const auto ra = buffer(p.A, (static_cast<uint64_t>(M - 1) * p.lda + p.K) * 4);
 
     // Rows past the last and depths past kend lie past the buffer's end.
     auto fetch = [&](float4 (&b)[NTR], uint32_t g0, uint32_t k, uint32_t kend) {
@@ -289,17 +298,31 @@ __global__ __launch_bounds__(64 * NTW) void gemv_f32_nt_kernel(F32Gemm p, uint32
 #pragma unroll
             for (int m = 0; m < M; ++m)
                 for (uint32_t i = tid; i < vecs; i += 64 * NTW)
-                    nt_lds[m * vecs + i] =
-                        kc + 4 * i < p.K ? *reinterpret_cast<const float4 *>(p.A + static_cast<uint64_t>(m) * p.lda + kc + 4 * i)
-                                         : make_float4(0.f, 0.f, 0.f, 0.f);
+                    load<4, 0>(ra, kc + 4 * i < p.K ? (m * p.lda + kc + 4 * i) * 4 : kOut, at + (m * vecs + i) * 4);
             __syncthreads();
             staged = chunk_k >= p.K;
         }
-        auto multiply = [&](const float4 (&b)[NTR], uint32_t kk) {
+        auto multiply = [&](float4 (&b)[NTR], uint32_t kk) {
             const float *ar = at + (kk - kc) + 4 * lane;
+            // a vector that K ends in (what follows it may be NaN)
+            const uint32_t left = p.K - (kk + 4 * lane);   // huge past K, where the loads gave zeros
+            const bool cut = (p.K & 3u) != 0 && kk + 256 > p.K;   // uniform
+            if (cut) {
+#pragma unroll
+                for (int r = 0; r < NTR; ++r) {
+                    if (left < 2) b[r].y = 0.0f;
+                    if (left < 3) b[r].z = 0.0f;
+                    if (left < 4) b[r].w = 0.0f;
+                }
+            }
 #pragma unroll
             for (int m = 0; m < M; ++m) {
-                const float4 a = *reinterpret_cast<const float4 *>(ar + m * chunk_k);
+                float4 a = *reinterpret_cast<const float4 *>(ar + m * chunk_k);
+                if (cut) {
+                    if (left < 2) a.y = 0.0f;
+                    if (left < 3) a.z = 0.0f;
+                    if (left < 4) a.w = 0.0f;
+                }
 #pragma unroll
                 for (int r = 0; r < NTR; ++r) {
                     float &t = acc[r * MP + m];
@@ -368,93 +391,106 @@ void launch_nt(hipStream_t s, const F32Gemm &p)
 
 namespace {
 
-bool aligned(const float *p, uint32_t ld, uint32_t n) { return ld % n == 0 && reinterpret_cast<uintptr_t>(p) % (4 * n) == 0; }
-
-// K ranges for workgroups of `cols` columns: the split that ends first, in
-// microseconds.  A workgroup alone on a CU takes 3 and its bytes at `cu`, or
-// its products at the CU's share of the matrix rate; a round of one per CU
-// takes no less than its bytes at `mem` (bytes per microsecond, measured on
-// this kernel's reads); a split costs the second launch that adds the ranges
-// (2.5).  N = K = 4096 at one range 28, at two 19.2, at four 15.5, at eight
-// 15.6; K = 11008 N = 4096 70, 42, 31.9, 32.3; N = 20000 64, 56, 51.7.
-void split(const F32Gemm &p, uint32_t cols, double cu, double mem, Plan &x)
+// Microseconds of the matrix-core kernel with 16 x.cb columns a workgroup, K in
+// the number of ranges that ends first.  A workgroup alone on a CU takes 2 and
+// its bytes at `cu` or its products at 0.2, 0.28 or 0.44e6 flops (wider ones
+// reuse more); a round of one per CU takes no less than its bytes at `mem`
+// (bytes per microsecond, measured on this kernel's reads); ranges cost the
+// second launch that adds them (3.5).  [K][N]
+// N = K = 4096 at one range 28, two 19.2, four 15.5, eight 15.6; K = 11008 N =
+// 4096 70, 42, 31.9, 32.3; K = 4096 N = 20000 64, 56, 51.7.
+double split(const F32Gemm &p, double cu, double mem, Plan &x)
 {
-    const uint32_t blocks = (p.N + cols - 1) / cols, cus = cu_count();
+    const uint32_t cols = 16 * x.cb, mg = p.M <= 16 ? 1 : p.M <= 32 ? 2 : 4, cus = cu_count();
+    const uint64_t tiles = static_cast<uint64_t>((p.N + cols - 1) / cols) * ((p.M + 16 * mg - 1) / (16 * mg));
     double best = 0.0;
     for (uint32_t s = 1; s == 1 || (s <= 16 && p.K / s >= 240); s *= 2) {
         const uint32_t k_per = ((p.K + s - 1) / s + 63) / 64 * 64;   // whole chunks
-        const double bytes = 4.0 * k_per * cols, flops = 32.0 * ((p.M + 15) / 16) * k_per * cols;
-        const double alone = 3.0 + std::max(bytes / cu, flops / 0.55e6);
-        const uint64_t wgs = static_cast<uint64_t>(blocks) * s;
+        const double bytes = 4.0 * k_per * cols, flops = 32.0 * mg * k_per * cols;
+        const double alone = 2.0 + std::max(bytes / cu, flops / (x.cb == 1 ? 0.2e6 : x.cb == 2 ? 0.28e6 : 0.44e6));
+        const uint64_t wgs = tiles * s;
         double t = static_cast<double>(wgs / cus) * std::max(alone, cus * bytes / mem);
         if (wgs % cus) t += std::max(alone, static_cast<double>(wgs % cus) * bytes / mem);
-        if (s > 1) t += 2.5;
+        if (s > 1) t += 3.5;
         if (s == 1 || t < best) {
             best = t;
             x.k_per = k_per;
             x.splits = (p.K + k_per - 1) / k_per;
         }
     }
+    return best;
 }
 
 // Which calls run here; the others keep the kernels of gemm_f32.hip.  Both
 // sides of each line measured on MI355X, weights from HBM (us, before -> here):
-//   [N][K] M <= 8: 128-column tiles of split products before.  4 x 4096 x
-//     32000 182 -> 87, x 4096 35 -> 14, 4 x 11008 x 4096 70 -> 35; below 8M
-//     weights the matrix-core kernel starts faster (8 x 1024 x 4096 14 -> 6.1
-//     against 8.3 with lanes along K).
-//   [N][K] M <= 32: 16 x 4096 x 4096 36 -> 24, x 32000 184 -> 145; 32 x 8192 x
-//     8192 101 -> 86.  M <= 64 only up to 8M weights: 64 x 2048 x 2048 18.5 ->
-//     15, but x 4096 x 11008 81 against 93.
+//   [N][K] M <= 8: 128-column tiles of split products before, or where rows are
+//     not 16-byte aligned the fp32 tile kernel.  4 x 4096 x 32000 182 -> 87, x
+//     4096 35 -> 14, 4 x 2047 x 11007 97 -> 19; below 8M weights the
+//     matrix-core kernel starts faster (8 x 1024 x 4096 14 -> 6.1 against 8.3
+//     with lanes along K).
+//   [N][K] M <= 32: 16 x 4096 x 4096 36 -> 22, x 32000 184 -> 145; 32 x 8192 x
+//     8192 101 -> 86, but x 11008 x 4096 71 against 75.  Aligned M <= 64 only up to 8M weights: 64 x 2048 x 2048
+//     18.5 -> 15, but x 4096 x 11008 81 against 93.
 //   [K][N] M <= 4: up to N = 4096 or 8M weights (4 x 4096 x 4096 19.8 -> 15.6,
-//     x 1024 x 1024 13 -> 6); wider, the split kernel's 1 KiB rows are as fast or faster (1 x
-//     4096 x 11008 31 against 35).
+//     x 1024 x 1024 13 -> 6); wider, or with unaligned rows from 2M weights, the
+//     split kernel's 1 KiB rows are as fast or faster (1 x 4096 x 11008 31
+//     against 35, 1 x 4096 x 4095 16.5 against 20).
 //   [K][N] M <= 8: up to N = 20480 (8 x 4096 x 16384 55 -> 42); wider, the wide
 //     kernel (8 x 4096 x 32000 84 against 87).
 //   [K][N] M <= 64: 16 x 4096 x 4096 39 -> 16.5, 32 x 4096 x 32000 195 -> 105,
 //     64 x 8192 x 8192 109 -> 82.
-//   Rows that are not 16-byte aligned ran on the fp32 tile kernel from M = 9 on
-//     (all of [N][K]): 16 x 4096 x 4095 [K][N] 70 -> 30, 32 x 1000 x 1001 23 ->
-//     9, 8 x 4095 x 4096 [N][K] 70 -> 56; narrow loads lose where many rows
-//     reuse a tile (64 x 2047 x 11007 105 against 149, [N][K] 32 x 1001 x 1000
-//     24 against 27).
+//   Aligned M > 64 only while the weights are so few that tiles of 128 leave the
+//     chip idle: 400 x 512 x 512 15 -> 8, 128 x 1024 x 1024 15 -> 10, 128 x 1024 x
+//     4096 24 -> 19; but 256 x 4096 x 1024 26 against 27, 200 x 2048 x 2048 24
+//     against 27.
+//   Unaligned rows ran on the fp32 tile kernel from M = 9 on: 16 x 4096 x 4095
+//     70 -> 21, 128 x 4095 x 4096 90 -> 47, 700 x 4095 x 4096 577 -> 228, 2000 x
+//     1000 x 1001 154 -> 48.  Its 128-row tiles win back many rows over a short K
+//     or, [N][K], wide weights (2048 x 333 x 4000 93 against 96; [N][K] 1000 x
+//     2047 x 11007 684 against 777).
 Plan plan(const F32Gemm &p)
 {
     Plan x;
-    // 32-bit offsets: the rows of A, and 64 rows of B
-    if (p.M > 64 || p.trans_a || p.cull || p.ktile_state || p.k_split_depth || p.ldb >= (1u << 22) ||
-        static_cast<uint64_t>(p.M) * p.lda >= (1u << 29))
+    // 32-bit offsets: 64 rows of A and of B
+    if (p.M > 2048 || p.trans_a || p.cull || p.ktile_state || p.k_split_depth || p.ldb >= (1u << 22) ||
+        p.lda >= (1u << 22))
         return x;
-    const bool a4 = aligned(p.A, p.lda, 4) && p.K % 4 == 0;
     const uint64_t weights = static_cast<uint64_t>(p.K) * p.N;
-    if (p.trans_b) {
-        const bool wide = a4 && aligned(p.B, p.ldb, 4);
-        if (wide && p.M <= 8 && weights >= (8u << 20)) {
-            x.kind = Plan::kLanes;
-            return x;
-        }
-        if (p.M > 16 && (!wide || (p.M > 32 && weights > (8u << 20)))) return x;
-        x.kind = Plan::kMatrix;
-        x.cb = p.M <= 8 || !wide || (p.M <= 16 && p.K <= 1024) ? 1 : 4;
-        split(p, 16 * x.cb, 25e3, 4.6e6, x);
+    auto even = [](const float *q, uint32_t ld) { return ld % 4 == 0 && reinterpret_cast<uintptr_t>(q) % 16 == 0; };
+    const bool even_b = even(p.B, p.ldb), even_ab = even_b && even(p.A, p.lda);
+    if (p.trans_b && p.M <= 8 && weights >= (8u << 20)) {
+        x.kind = Plan::kLanes;
         return x;
     }
-    x.cb = p.N % 4 == 0 && aligned(p.B, p.ldb, 4) ? 4 : p.N % 2 == 0 && aligned(p.B, p.ldb, 2) ? 2 : 1;
-    const bool small = p.M <= 32 && p.K <= 1024 && weights <= (2u << 20);
-    if (!small) {
-        const uint32_t widest = p.M <= 4 ? (x.cb != 4 ? 0 : weights <= (8u << 20) ? UINT32_MAX : 4096)
-                                : p.M <= 8 ? (x.cb == 4 ? 20480 : x.cb == 2 ? 8192 : 0)
-                                : p.M <= 32 || x.cb == 4 ? UINT32_MAX : 8192;
-        if (p.N > widest) return x;
-    } else {
-        x.cb = 1;   // a grid of 16-column workgroups is done before a second launch would start
+    if (even_ab) {   // the split-bf16 tiles' ground from 65 rows on, and in part before
+        if (p.M > 64 && weights > (p.M <= 128 ? 9u << 19 : p.M <= 1024 ? 1u << 20 : 0)) return x;
+        if (p.trans_b && (p.M > 32 ? weights > (8u << 20) : p.M > 16 && p.K > 8192)) return x;
+    } else if (p.M > (p.trans_b ? 768 : 1024)) {
+        if (p.K < 512 || (p.trans_b && weights > (17u << 20))) return x;
+    }
+    if (!p.trans_b) {
+        if (p.M <= 4 && weights > (even_b ? 8u << 20 : 2u << 20) && !(even_b && p.N <= 4096)) return x;
+        if (p.M <= 8 && p.N > 20480) return x;
     }
     x.kind = Plan::kMatrix;
-    if (small) {
-        x.k_per = (p.K + 63) / 64 * 64;
-        return x;
+    // 64 columns a workgroup read the longest runs and share A the most; narrower
+    // ones fill the chip where the output is small, and [N][K] up to 16 rows,
+    // whose runs do not grow with the columns, likewise below N = 8192 (16 x 4096
+    // x 4096 22 against 24).
+    static const double kRate[2][3][2] = {{{18e3, 2.8e6}, {30e3, 5.0e6}, {35e3, 6.0e6}},    // [K][N]
+                                          {{25e3, 3.4e6}, {25e3, 3.5e6}, {25e3, 3.6e6}}};   // [N][K]
+    const bool small = weights <= (4u << 20);
+    const int most = !small && p.trans_b && p.M <= 16 && p.N < 8192 ? 0 : 2;
+    double best = 0.0;
+    for (int i = most; i >= (small ? 0 : most); --i) {
+        Plan y = x;
+        y.cb = 1 << i;
+        const double t = split(p, kRate[p.trans_b][i][0], kRate[p.trans_b][i][1], y);
+        if (i == most || t < best) {
+            best = t;
+            x = y;
+        }
     }
-    split(p, 16 * x.cb, x.cb == 4 ? 35e3 : x.cb == 2 ? 30e3 : 25e3, x.cb == 4 ? 6.0e6 : x.cb == 2 ? 5.0e6 : 4.0e6, x);
     return x;
 }
 
@@ -484,18 +520,10 @@ void skinny_f32(hipStream_t s, const F32Gemm &p, float *ws)
         }
         return;
     }
-    const bool a4 = aligned(p.A, p.lda, 4) && p.K % 4 == 0, b4 = aligned(p.B, p.ldb, 4);
     auto rows = [&](auto mg) {
         constexpr int MG = decltype(mg)::value;
-        auto depths = [&](auto va) {
-            constexpr int VA = decltype(va)::value;
-            if (p.trans_b) launch_matrix<MG, true, VA, VA>(s, p, x, ws);
-            else if (x.cb == 4) launch_matrix<MG, false, VA, 4>(s, p, x, ws);
-            else if (x.cb == 2) launch_matrix<MG, false, VA, 2>(s, p, x, ws);
-            else launch_matrix<MG, false, VA, 1>(s, p, x, ws);
-        };
-        if (a4 && (b4 || !p.trans_b)) depths(std::integral_constant<int, 4>{});
-        else depths(std::integral_constant<int, 1>{});
+        if (p.trans_b) launch_matrix<MG, true>(s, p, x, ws);
+        else launch_matrix<MG, false>(s, p, x, ws);
     };
     if (p.M <= 16) rows(std::integral_constant<int, 1>{});
     else if (p.M <= 32) rows(std::integral_constant<int, 2>{});

@@ -599,7 +599,10 @@ def test_matmul_f32_strided_operands(gpu, M, K, N, ta, tb):
     # [K][N]: 64, 32 and 16 columns a workgroup, with K split and not, widths left over
     (4, 3000, 132, 0, 0, 0), (16, 4100, 68, 0, 4, 4), (33, 1999, 200, 0, 1, 0), (64, 2048, 4, 0, 0, 0),
     (8, 2048, 70, 0, 0, 2), (31, 4097, 34, 0, 0, 0), (12, 1500, 1503, 0, 0, 2), (64, 1030, 17, 0, 0, 0),
-    (2, 513, 1000, 0, 0, 0), (32, 15, 7, 0, 0, 0)])
+    (2, 513, 1000, 0, 0, 0), (32, 15, 7, 0, 0, 0),
+    # unaligned rows with lanes along K (a last vector that K ends in), and more than 64 rows
+    (2, 8193, 1026, 1, 0, 0), (8, 8450, 1001, 1, 1, 3), (77, 1003, 1001, 0, 0, 0), (130, 514, 67, 1, 0, 1),
+    (700, 513, 129, 0, 1, 0), (66, 1024, 512, 0, 0, 0), (1100, 515, 300, 0, 2, 1), (3, 3, 2, 0, 0, 0)])
 def test_matmul_f32_few_rows(gpu, M, K, N, tb, lda_pad, ldb_pad):
     """Few rows (skinny_f32.hip) at the edges of its tiles and rules.  Every
     product and sum is f32, in chains of at most K / 16 terms: the error is
