@@ -524,7 +524,9 @@ void exec_matmul_i8(vnpu_device_t *dev, vnpu_stream_t *s, const vnpu_matmul_i8_a
     const size_t c_bytes = span(in.M, in.N, p.ldc, 4);
     p.C = p.ldc != in.N ? sg.inout(in.C, c_bytes) : sg.out(in.C, c_bytes);
 
-    if (k::gemv_i8_takes(in.M, in.N))
+    if (k::direct_i8_takes(p))
+        k::direct_i8(s->hip, p);
+    else if (in.M <= k::kGemvMaxRows)
         k::gemv_i8(s->hip, p);
     else
         k::gemm_i8(s->hip, p, static_cast<int8_t *>(s->ensure_workspace(k::gemm_i8_ws_bytes(p))));

@@ -24,7 +24,7 @@
 //   * the activations (M x K int8, tiny) are staged in LDS as [k/16][m][16]
 //     (dynamic LDS sized to the chunk actually used), so lane kg reads its
 //     16 bytes of every row with one ds_read_b128 per row; the matrix-core
-//     kernel for up to 16 rows instead reads them from global memory with
+//     kernel instead reads them from global memory with
 //     each weight block when the rows are 16-byte aligned
 //     (gemv_i8_mfma_direct);
 //   * v_dot4_i32_i8 (4 per 16 bytes per row) accumulates in int32 for up
@@ -230,17 +230,13 @@ __global__ __launch_bounds__(64 * W) void gemv_i8_kernel(I8Gemm p, uint32_t chun
     epi.template store<W, T, M>(p, red, nt0, NT, tid);
 }
 
-// The same stream for 3..64 rows with the int8 matrix core doing the math: a
+// The same stream for 4..8 rows with the int8 matrix core doing the math: a
 // packed 1 KiB weight block is exactly the B operand of one
 // v_mfma_i32_16x16x64_i8 (lane 16kg + c holds k 16kg..16kg+15 of column c),
-// and the A operand is the staged activations (lane l: row l%16 of a group of
-// 16 rows, the same 16 k; rows past M are zero).  One MFMA per block and row
-// group replaces 4M v_dot4 and M ds_read_b128 per lane, which at M = 8 made
-// the VALU the bottleneck.  The 16 x 16 result leaves row 4(l/16) + i, column
-// l%16 in lane l, register i.  M is the row capacity: the kernels for up to
-// 8 rows are built per row count, those for 16, 32 and 64 take any p.M up to
-// it (the staged layout uses p.M; rows past it are zero and not stored), and
-// above 16 rows the wave sums go through the activation LDS once it is free.
+// and the A operand is the staged activations (lane l: row l%16, the same 16 k;
+// rows past M are zero).  One MFMA per block replaces 4M v_dot4 and M
+// ds_read_b128 per lane, which at M = 8 made the VALU the bottleneck.  The
+// 16 x 16 result leaves row 4(l/16) + i, column l%16 in lane l, register i.
 template <int M, int W, int U, int T>
 __global__ __launch_bounds__(64 * W) void gemv_i8_mfma(I8GemmPair ps, uint32_t grid0, uint32_t chunk_k)
 {
@@ -249,13 +245,10 @@ __global__ __launch_bounds__(64 * W) void gemv_i8_mfma(I8GemmPair ps, uint32_t g
     const bool second = blockIdx.x >= grid0;
     const I8Gemm &p = ps.p[second ? 1 : 0];
     const uint32_t bx = second ? blockIdx.x - grid0 : blockIdx.x;
-    static_assert(M <= 64, "at most four 16-row groups");
-    constexpr int MG = (M + 15) / 16;
+    static_assert(M <= 16, "one 16-row group");
     typedef int v4i __attribute__((ext_vector_type(4)));
-    extern __shared__ __attribute__((aligned(16))) int8_t a_lds[];  // [chunk_k/16][Mr][16]
-    __shared__ int red_s[M <= 16 ? W * T * M * 16 : 1];
-    // rows present: the template's count up to 8 rows, else the call's
-    const uint32_t Mr = M <= 8 ? static_cast<uint32_t>(M) : ps.p[0].M;
+    extern __shared__ __attribute__((aligned(16))) int8_t a_lds[];  // [chunk_k/16][M][16]
+    __shared__ int red[W][T][M][16];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -265,11 +258,9 @@ __global__ __launch_bounds__(64 * W) void gemv_i8_mfma(I8GemmPair ps, uint32_t g
     const uint32_t KT = p.Kp >> 6;
     const bool vec_a = ((p.lda & 15u) == 0) && ((reinterpret_cast<uintptr_t>(p.A) & 15u) == 0);
 
-    v4i acc[MG][T];
+    v4i acc[T];
 #pragma unroll
-    for (int g = 0; g < MG; ++g)
-#pragma unroll
-        for (int t = 0; t < T; ++t) acc[g][t] = (v4i){0, 0, 0, 0};
+    for (int t = 0; t < T; ++t) acc[t] = (v4i){0, 0, 0, 0};
     const EpiOperands<T * M * 16, 64 * W> epi(p, nt0, M, tid);
 
     for (uint32_t kc = 0; kc < p.Kp; kc += chunk_k) {
@@ -296,9 +287,9 @@ __global__ __launch_bounds__(64 * W) void gemv_i8_mfma(I8GemmPair ps, uint32_t g
             for (int t = 0; t < T; ++t) bc[u][t] = ld(t, u);
 
         if (kc) __syncthreads();  // previous chunk fully consumed
-        const uint32_t chunks = (kt1 - kt0) * 4 * Mr;
+        const uint32_t chunks = (kt1 - kt0) * 4 * M;
         for (uint32_t i = tid; i < chunks; i += 64 * W) {
-            const uint32_t m = i % Mr, k16 = i / Mr;
+            const uint32_t m = i % M, k16 = i / M;
             const uint32_t k = kc + k16 * 16;
             const int8_t *src = p.A + static_cast<uint64_t>(m) * p.lda + k;
             int4 v;
@@ -313,7 +304,7 @@ __global__ __launch_bounds__(64 * W) void gemv_i8_mfma(I8GemmPair ps, uint32_t g
                 for (int j = 0; j < 16; ++j) u.b[j] = (k + j < p.K) ? src[j] : 0;
                 v = u.v;
             }
-            *reinterpret_cast<int4 *>(a_lds + (k16 * Mr + m) * 16) = v;
+            *reinterpret_cast<int4 *>(a_lds + (k16 * M + m) * 16) = v;
         }
         __syncthreads();
 
@@ -325,15 +316,11 @@ __global__ __launch_bounds__(64 * W) void gemv_i8_mfma(I8GemmPair ps, uint32_t g
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const uint32_t ktl = first + W * min(i + u, cnt - 1) - kt0;
+                v4i a = (v4i){0, 0, 0, 0};
+                if (row < M) a = *reinterpret_cast<const v4i *>(a_lds + ((ktl * 4 + kg) * M + row) * 16);
 #pragma unroll
-                for (int g = 0; g < MG; ++g) {
-                    const uint32_t r = 16 * g + row;
-                    v4i a = (v4i){0, 0, 0, 0};
-                    if (r < Mr) a = *reinterpret_cast<const v4i *>(a_lds + ((ktl * 4 + kg) * Mr + r) * 16);
-#pragma unroll
-                    for (int t = 0; t < T; ++t)
-                        acc[g][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, bc[u][t], acc[g][t], 0, 0, 0);
-                }
+                for (int t = 0; t < T; ++t)
+                    acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, bc[u][t], acc[t], 0, 0, 0);
             }
 #pragma unroll
             for (int u = 0; u < U; ++u)
@@ -342,20 +329,14 @@ __global__ __launch_bounds__(64 * W) void gemv_i8_mfma(I8GemmPair ps, uint32_t g
         }
     }
 
-    // Lane l holds rows 16g + 4(l/16) + i of column l%16; sum the waves in LDS
-    // (above 16 rows in the activation area, once every wave is done with it).
-    if constexpr (M > 16) __syncthreads();
-    auto &red = *reinterpret_cast<int (*)[W][T][M][16]>(M <= 16 ? static_cast<void *>(red_s)
-                                                                 : static_cast<void *>(a_lds));
+    // lane l holds rows 4(l/16) + i of column l%16
 #pragma unroll
-    for (int g = 0; g < MG; ++g)
+    for (int t = 0; t < T; ++t)
 #pragma unroll
-        for (int t = 0; t < T; ++t)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int m = 16 * g + 4 * kg + i;
-                if (m < M) red[wave][t][m][row] = acc[g][t][i];
-            }
+        for (int i = 0; i < 4; ++i) {
+            const int m = 4 * kg + i;
+            if (m < M) red[wave][t][m][row] = acc[t][i];
+        }
     __syncthreads();
     epi.template store<W, T, M>(p, red, nt0, NT, tid);
 }
@@ -365,7 +346,7 @@ __global__ __launch_bounds__(64 * W) void gemv_i8_mfma(I8GemmPair ps, uint32_t g
 // for each k block alongside that block's weights (one A load serves the T
 // strips), so no staging pass and barrier sit between the first weight loads
 // and the first MFMA.  Needs 16-byte aligned rows (lda % 16 == 0,
-// K % 16 == 0); rows past p.M and k past K read as zeros through the
+// K % 16 == 0); rows past M and k past K read as zeros through the
 // buffer's range check.
 template <int M, int W, int U, int T>
 __global__ __launch_bounds__(64 * W) void gemv_i8_mfma_direct(I8GemmPair ps, uint32_t grid0)
@@ -376,7 +357,6 @@ __global__ __launch_bounds__(64 * W) void gemv_i8_mfma_direct(I8GemmPair ps, uin
     const uint32_t nt0 = (second ? blockIdx.x - grid0 : blockIdx.x) * T;
     typedef int v4i __attribute__((ext_vector_type(4)));
     __shared__ int red[W][T][M][16];
-    const uint32_t Mr = M <= 8 ? static_cast<uint32_t>(M) : p.M;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -398,8 +378,8 @@ __global__ __launch_bounds__(64 * W) void gemv_i8_mfma_direct(I8GemmPair ps, uin
     // A: one buffer over the Mr rows; the lane's offset is past the end for a
     // row past Mr, a block past the wave's last or k past K
     const auto ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(p.A), 0,
-                                                      static_cast<int>((Mr - 1) * p.lda + p.K), kBufferWord3);
-    const bool row_live = static_cast<uint32_t>(row) < Mr;
+                                                      static_cast<int>((M - 1) * p.lda + p.K), kBufferWord3);
+    const bool row_live = row < M;
     const uint32_t a_row = row_live ? row * p.lda : 0u;
     auto ldb = [&](int t, uint32_t i) {
         return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rw[t], i * W * 1024 + lane * 16, 0,
@@ -516,31 +496,23 @@ template <int M>
 void launch_mfma_pair(hipStream_t s, const I8GemmPair &ps, int variant, uint32_t grid0, uint32_t grid1,
                       uint32_t chunk_k)
 {
-    // above 16 rows the wave sums ([W][T][M][16] int32, 64 W T M bytes; W T =
-    // 24 for <8,2,3>, 16 in the other variants) reuse the activation LDS
-    const size_t wt = variant == 3 ? 24u : 16u;
-    const size_t lds = std::max<size_t>(static_cast<size_t>(chunk_k) * M, M > 16 ? 64u * wt * M : 0u);
+    const size_t lds = static_cast<size_t>(chunk_k) * M;
     const dim3 grid(grid0 + grid1);
-    const bool direct = M <= 16 && direct_a(ps.p[0]) && (grid1 == 0 || direct_a(ps.p[1]));
+    const bool direct = direct_a(ps.p[0]) && (grid1 == 0 || direct_a(ps.p[1]));
     if (direct) {
-        if constexpr (M <= 16) {
-            if (variant == 0)
-                gemv_i8_mfma_direct<M, 4, 4, 4><<<grid, 256, 0, s>>>(ps, grid0);
-            else if (variant == 1)
-                gemv_i8_mfma_direct<M, 8, 2, 2><<<grid, 512, 0, s>>>(ps, grid0);
-            else if (variant == 3)
-                gemv_i8_mfma_direct<M, 8, 2, 3><<<grid, 512, 0, s>>>(ps, grid0);
-            else
-                gemv_i8_mfma_direct<M, 16, 2, 1><<<grid, 1024, 0, s>>>(ps, grid0);
-        }
+        if (variant == 0)
+            gemv_i8_mfma_direct<M, 4, 4, 4><<<grid, 256, 0, s>>>(ps, grid0);
+        else if (variant == 1)
+            gemv_i8_mfma_direct<M, 8, 2, 2><<<grid, 512, 0, s>>>(ps, grid0);
+        else if (variant == 3)
+            gemv_i8_mfma_direct<M, 8, 2, 3><<<grid, 512, 0, s>>>(ps, grid0);
+        else
+            gemv_i8_mfma_direct<M, 16, 2, 1><<<grid, 1024, 0, s>>>(ps, grid0);
     } else if (variant == 0) {
-        if (M > 16) lds_optin<gemv_i8_mfma<M, 4, 4, 4>>();
         gemv_i8_mfma<M, 4, 4, 4><<<grid, 256, lds, s>>>(ps, grid0, chunk_k);
     } else if (variant == 1) {
-        if (M > 16) lds_optin<gemv_i8_mfma<M, 8, 2, 2>>();
         gemv_i8_mfma<M, 8, 2, 2><<<grid, 512, lds, s>>>(ps, grid0, chunk_k);
     } else if (variant == 3) {
-        if (M > 16) lds_optin<gemv_i8_mfma<M, 8, 2, 3>>();
         gemv_i8_mfma<M, 8, 2, 3><<<grid, 512, lds, s>>>(ps, grid0, chunk_k);
     } else {
         lds_optin<gemv_i8_mfma<M, 16, 2, 1>>();
@@ -610,13 +582,7 @@ void gemv_i8(hipStream_t s, const I8Gemm &p)
     case 5: launch_m<5>(s, p); break;
     case 6: launch_m<6>(s, p); break;
     case 7: launch_m<7>(s, p); break;
-    case 8: launch_m<8>(s, p); break;
-    default:
-        // 9..64 rows: the matrix-core kernel with a row capacity of 16, 32 or 64
-        if (p.M <= 16) launch_m<16>(s, p);
-        else if (p.M <= 32) launch_m<32>(s, p);
-        else if (p.M <= kGemvMaxRows) launch_m<64>(s, p);
-        break;
+    default: launch_m<8>(s, p); break;
     }
 }
 

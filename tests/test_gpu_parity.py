@@ -326,6 +326,51 @@ def test_matmul_i8_few_rows(gpu, M, K, N):
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("M,K,N,lda_pad,off,ldc_pad", [
+    # every workgroup shape (16 x 16 to 64 x 64), whole and with a row, a column or a depth over
+    (16, 4096, 4096, 0, 0, 0), (32, 4096, 4096, 0, 0, 0), (64, 4096, 4096, 0, 0, 0), (96, 4096, 4096, 0, 0, 0),
+    (200, 4096, 4096, 0, 0, 0), (200, 1024, 2000, 0, 0, 5), (331, 1376, 5003, 0, 0, 0), (65, 4160, 4111, 0, 0, 0),
+    (17, 2112, 2050, 16, 0, 0), (33, 11072, 2063, 0, 0, 1), (49, 4096, 9001, 16, 0, 0), (130, 130, 4100, 2, 0, 0),
+    # rows from any byte: lda and the first row at 1, 2 and 3 past a dword
+    (9, 65, 17, 0, 0, 0), (63, 1001, 4100, 0, 1, 0), (150, 1001, 4100, 0, 2, 3), (40, 515, 300, 2, 3, 0),
+    (16, 4095, 33, 0, 3, 0), (700, 129, 1001, 0, 1, 0), (24, 1030, 8200, 0, 2, 0), (12, 4096, 800, 0, 3, 0),
+    # the smallest, less than a pair of blocks, fewer blocks than waves
+    (9, 1, 1, 0, 0, 0), (64, 3, 5, 0, 1, 0), (100, 64, 16, 0, 4, 0), (11, 200, 40, 0, 0, 0),
+    # weights past the last-level cache, one row tile; five to eight rows of wide weights
+    (5, 1000, 16400, 0, 0, 0), (8, 4096, 24700, 0, 0, 0), (7, 333, 20001, 0, 1, 2), (28, 4096, 24700, 0, 0, 0),
+    (60, 4160, 24577, 0, 0, 0)])
+def test_matmul_i8_direct(gpu, M, K, N, lda_pad, off, ldc_pad):
+    """Rows between the GEMV and the staged tiles, and rows of any alignment
+    (direct_i8.hip): bit-exact against the float64 accumulator, which is the exact
+    int32 one, and without bias each of the two products rounds once."""
+    rng = np.random.default_rng(M * 7 + K * 3 + N + off)
+    lda, ldc = K + lda_pad, N + ldc_pad
+    A = rng.integers(-128, 128, size=off + (M - 1) * lda + K).astype(np.int8)   # ends with the last row
+    rows = np.lib.stride_tricks.as_strided(A[off:], (M, K), (lda, 1))
+    B = rng.integers(-128, 128, size=(K, N)).astype(np.int8)
+    sa = ((rng.random(M) + 0.5) / 127).astype(np.float32)
+    sb = ((rng.random(N) + 0.5) / 127).astype(np.float32)
+    bias = rng.standard_normal(N).astype(np.float32)
+    w = gpu.pack(B, K, N, scales=sb)
+    ba, bsa, bbias = gpu.upload(A), gpu.upload(sa), gpu.upload(bias)
+    c0 = np.full((M, ldc), 7.0, np.float32)
+    bc, bd = gpu.upload(c0), gpu.upload(c0)
+    try:
+        gpu.run(abi.OP_MATMUL_I8, A=ba.ptr + off, B=w, C=bc, M=M, K=K, N=N, lda=lda, ldc=ldc, scale_a=bsa)
+        gpu.run(abi.OP_MATMUL_I8, A=ba.ptr + off, B=w, C=bd, M=M, K=K, N=N, lda=lda, ldc=ldc, bias=bbias,
+                epilogue=abi.EPI_RELU)
+        got, got_bias = gpu.download(bc, np.float32, (M, ldc)), gpu.download(bd, np.float32, (M, ldc))
+    finally:
+        for b in (ba, bsa, bbias, bc, bd):
+            gpu.free(b)
+        gpu.release_packed(w)
+    acc = (rows.astype(np.float64) @ B.astype(np.float64)).astype(np.float32)
+    want = (acc * sa[:, None]) * sb[None, :]
+    assert np.array_equal(got[:, :N].view(np.uint32), want.view(np.uint32))
+    assert np.array_equal(got_bias[:, :N], np.maximum(acc * sb[None, :] + bias[None, :], 0))
+    assert np.all(got[:, N:] == 7.0) and np.all(got_bias[:, N:] == 7.0)
+
+
 @pytest.mark.parametrize("M", [1, 6, 40])
 def test_matmul_i8_accumulator_exact(gpu, M):
     # scale 1 everywhere: C == (float)acc exactly while |acc| < 2^24
