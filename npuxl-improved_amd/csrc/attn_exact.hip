@@ -1025,10 +1025,14 @@ void launch_decode(hipStream_t s, const Attn &a, float *ws)
         c.batch = n;
         c.heads = 1;
         const uint32_t tiles = (a.seq_k + XB - 1) / XB;
-        // One tile a wave until there are four waves a CU: the waves of a short
-        // context would otherwise take their tiles in turn on an idle chip.
-        const uint32_t tpw = std::min<uint32_t>(DTPW, std::max<uint32_t>(1, tiles * n / (4 * cu_count())));
-        attn_dec_scores<D><<<dim3((tiles + tpw - 1) / tpw, n), 64, dec_scores_lds<D>(a.seq_q), s>>>(c, ws, pitch, tpw);
+        // As many tiles a wave as make one round of the workgroups that LDS lets the
+        // CUs hold: with more, the waves of a short context take their tiles in turn
+        // on an idle chip, with fewer a second round runs part empty (64 heads x 2
+        // rows of 4000 keys at head_dim 128: three a wave 99.9 us, four 95).
+        const size_t lds = dec_scores_lds<D>(a.seq_q);
+        const uint64_t slots = 160 * 1024 / lds * cu_count();
+        const uint32_t tpw = static_cast<uint32_t>(std::min<uint64_t>(DTPW, (static_cast<uint64_t>(tiles) * n + slots - 1) / slots));
+        attn_dec_scores<D><<<dim3((tiles + tpw - 1) / tpw, n), 64, lds, s>>>(c, ws, pitch, tpw);
         attn_dec_chain<D><<<dim3(n * a.seq_q, XL<D>::NM), 64, kDecLds, s>>>(c, ws, pitch);
     }
 }
@@ -1055,17 +1059,26 @@ bool attention_exact_supported(const Attn &a)
     if (a.head_dim % 8 || a.head_dim > 128) return false;
     for (const float *p : {a.Q, a.K, a.V, static_cast<const float *>(a.O)})
         if (reinterpret_cast<uintptr_t>(p) % 16) return false;
+    // a handful of keys and few rows: the general kernel's one pass over them
+    // (4 heads of 32 x 4 rows, 8 keys, head_dim 80 5.4 us against 6.5)
+    if (a.seq_k <= 12 && static_cast<uint64_t>(a.batch) * a.heads * a.seq_q <= 1024) return false;
     return a.seq_q > 4 || dec_scores_bytes(a) <= kDecScoreCap;
 }
 
 bool attention_exact_decodes(const Attn &a)
 {
-    if (a.seq_q <= 4) return true;
-    // A few more rows behind a long context (the check of drafted tokens), as
-    // long as the rows' chains fit the chip at once: 32 heads x 5 rows x 4000
-    // keys at head_dim 128 100 us against 240 with 32-row workgroups; at 300
-    // keys, or more rows, the two launches and the repeated reads of V lose.
+    // A row's chains cost two launches and read V once per row; 32-row workgroups
+    // read it once but leave most of their rows idle.  Few keys go to the latter
+    // (32 heads x 4 rows of 40 keys 9.0 -> 6.2 us, 1 row 7.3 -> 6.2), and so do two
+    // to four rows of so many heads that the chains do not fit the chip at once
+    // (256 heads x 4 rows of 160 keys at head_dim 128 40.0 -> 18.2 us).
     const uint64_t chains = static_cast<uint64_t>(a.batch) * a.heads * a.seq_q * ((a.head_dim + 63) / 64);
+    if (a.seq_k < std::max(64u, 32 * a.seq_q)) return false;
+    if (a.seq_q <= 4)   // (two rows of a long context: 258 us against 267 for 256 heads x 4000 keys)
+        return a.seq_q == 1 || chains <= 2 * cu_count() || (a.seq_q == 2 && a.seq_k >= 2048);
+    // A few more rows behind a long context (the check of drafted tokens), as
+    // long as the chains fit: 32 heads x 5 rows x 4000 keys at head_dim 128 100 us
+    // against 240 with 32-row workgroups; at 300 keys, or more rows, they lose.
     return a.seq_q <= kDecMaxRows && a.seq_k >= 1024 && chains <= 2 * cu_count() && dec_scores_bytes(a) <= kDecScoreCap;
 }
 

@@ -232,6 +232,30 @@ def test_attention_reference_order_prefill_shapes(exact_gpu, b, h, sq, sk, d, ca
     assert bits(got, block_oracle.attention_threaded(Q, K, V, causal, mask=M, avx2=True))
 
 
+@pytest.mark.parametrize("d", [64, 80, 128])
+@pytest.mark.parametrize("b,h,sq,sk,causal,mask", [
+    (2, 3, 1, 63, 1, None), (2, 3, 1, 64, 0, "normal"),        # one row: 32-row workgroups below 64 keys
+    (1, 2, 4, 127, 0, "inf"), (1, 2, 4, 128, 1, None),         # and four rows below 128
+    (1, 3, 2, 12, 1, None), (1, 3, 3, 13, 0, "row"),           # a handful of keys
+    (9, 32, 2, 200, 1, None),                                  # rows of many heads
+    (2, 33, 1, 2000, 0, None)])                                # scores: two tiles a wave, the last one alone
+def test_attention_reference_order_few_rows(exact_gpu, b, h, sq, sk, d, causal, mask):
+    """One to four rows on each side of the lines between the chains, the 32-row
+    workgroups and the general kernel: the reference order, bit for bit."""
+    Q = RNG.standard_normal((b, h, sq, d)).astype(np.float32)
+    K = RNG.standard_normal((b, h, sk, d)).astype(np.float32)
+    V = RNG.standard_normal((b, h, sk, d)).astype(np.float32)
+    M = None
+    if mask:
+        M = RNG.standard_normal((b, h, sq, sk)).astype(np.float32)
+        if mask == "inf":
+            M[RNG.random(M.shape) < 0.3] = -np.inf
+        if mask == "row":
+            M[:, :, 0, :] = -np.inf                            # a row with no key left
+    got = g.attention(exact_gpu, Q, K, V, M, causal)
+    assert bits(got, block_oracle.attention_threaded(Q, K, V, causal, mask=M, avx2=True))
+
+
 @pytest.mark.parametrize("d", [8, 32, 40, 56, 80, 88, 96, 120])
 @pytest.mark.parametrize("b,h,sq,sk,causal,mask", [
     (2, 2, 1, 129, 1, None), (1, 3, 4, 300, 0, "normal"),      # decode: one tile per scores wave, ragged keys
