@@ -442,7 +442,8 @@ __global__ __launch_bounds__(64 * W) void gemv_i8_mfma_direct(I8GemmPair ps, uin
 //     workgroup per strip, at most 256 workgroups) sixteen waves with four
 //     (M = 1) or two blocks (M=1 N=4096 5.2 -> 4.8 us).
 //   * matrix-core kernel (M >= 5; at three and four rows v_dot4 is as fast):
-//     from 1024 strips four strips per workgroup so one staged activation
+//     from 1024 strips (a pair, or with an ADD in the store: others take
+//     direct_i8.hip there) four strips per workgroup so one staged activation
 //     chunk serves four weight streams, <W,U,T> = <4,4,4>; 512-1023 strips
 //     two strips per workgroup, <8,2,2> (M=8 N=11008 11.9 -> 11.1 us with
 //     <8,4,1>, then N=12288 11.8 -> 11.5 us and N=8200 10.6 -> 9.9 us with two
@@ -452,7 +453,7 @@ __global__ __launch_bounds__(64 * W) void gemv_i8_mfma_direct(I8GemmPair ps, uin
 //     strips per workgroup, <8,2,3>, so no CU streams twice the bytes of
 //     another (768 strips at N = 12288: 384 workgroups of two strips leave
 //     half the CUs with two of them).  M=8 N=12288 11.8 -> 11.3 us, N=11008
-//     11.4 -> 10.7 us, M=16 N=12288 14.1 -> 12.6 us; the pair grids keep two
+//     11.4 -> 10.7 us; the pair grids keep two
 //     strips (two problems of 688 strips balance no better with three).
 int mfma_variant(uint32_t NT) { return NT >= 1024 ? 0 : NT >= 512 ? 1 : 2; }
 int mfma_variant_one(uint32_t NT)
