@@ -1051,14 +1051,20 @@ void with_tile(uint32_t head_dim, F &&f)
     else f(std::integral_constant<int, 128>{});
 }
 
+bool aligned16(const Attn &a)
+{
+    for (const float *p : {a.Q, a.K, a.V, static_cast<const float *>(a.O)})
+        if (reinterpret_cast<uintptr_t>(p) % 16) return false;
+    return true;
+}
+
 }  // namespace
 
 bool attention_exact_supported(const Attn &a)
 {
     if (a.head_dim == 64 || a.head_dim == 128) return true;
     if (a.head_dim % 8 || a.head_dim > 128) return false;
-    for (const float *p : {a.Q, a.K, a.V, static_cast<const float *>(a.O)})
-        if (reinterpret_cast<uintptr_t>(p) % 16) return false;
+    if (!aligned16(a)) return false;
     // a handful of keys and few rows: the general kernel's one pass over them
     // (4 heads of 32 x 4 rows, 8 keys, head_dim 80 5.4 us against 6.5)
     if (a.seq_k <= 12 && static_cast<uint64_t>(a.batch) * a.heads * a.seq_q <= 1024) return false;
@@ -1073,6 +1079,7 @@ bool attention_exact_decodes(const Attn &a)
     // to four rows of so many heads that the chains do not fit the chip at once
     // (256 heads x 4 rows of 160 keys at head_dim 128 40.0 -> 18.2 us).
     const uint64_t chains = static_cast<uint64_t>(a.batch) * a.heads * a.seq_q * ((a.head_dim + 63) / 64);
+    if (a.seq_q <= 4 && !aligned16(a)) return true;   // the chains read Q and write O by dwords
     if (a.seq_k < std::max(64u, 32 * a.seq_q)) return false;
     if (a.seq_q <= 4)   // (two rows of a long context: 258 us against 267 for 256 heads x 4000 keys)
         return a.seq_q == 1 || chains <= 2 * cu_count() || (a.seq_q == 2 && a.seq_k >= 2048);
