@@ -712,7 +712,6 @@ __global__ __launch_bounds__(XT) void attn_exact_coop_kernel(Attn a)
         const bool odd = g16 & 1;              // l is of row c32
         l = (odd ? live[1] : live[0]) ? l * (odd ? alpha[1] : alpha[0]) + psum : l;
     }
-    if (!writes) return;
 
     // oacc[4q + i]: element 32 wave + 16(q / 2) + 4 g16 + i of row 16(q % 2) + c16.
     const float l0 = __shfl(l, c16, 64), l1 = __shfl(l, 16 + c16, 64);
@@ -727,7 +726,12 @@ __global__ __launch_bounds__(XT) void attn_exact_coop_kernel(Attn a)
         const bool stored = q0 + 16 * odd + c16 < sq && e0 + 16 * (r >> 3) < hd;
         bad |= stored && ((o != o) || (o == 0.0f && (odd ? l1 : l0) > 0.0f));
     }
-    if (__ballot(bad) == 0) {
+    // A row is recomputed whole, by one wave, before any wave stores a part of
+    // it: O may be Q.  The maxima in Mx were read before the last barrier.
+    const bool any = __ballot(bad) != 0;
+    if (lane == 0) Mx[wave] = any ? 1.0f : 0.0f;
+    lds::block_barrier();
+    if (Mx[0] + Mx[1] + Mx[2] + Mx[3] == 0.0f) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const uint32_t row = q0 + 16 * (q & 1) + c16, e = e0 + 16 * (q >> 1);
@@ -736,7 +740,7 @@ __global__ __launch_bounds__(XT) void attn_exact_coop_kernel(Attn a)
                     make_float4(oacc[4 * q], oacc[4 * q + 1], oacc[4 * q + 2], oacc[4 * q + 3]);
         }
     } else {
-        for (uint32_t j = 0; j < XQW && q0 + j < sq; ++j) exact_row_wave<D>(a, bh, q0 + j, lane);
+        for (uint32_t j = wave; j < XQW && q0 + j < sq; j += 4) exact_row_wave<D>(a, bh, q0 + j, lane);
     }
 }
 

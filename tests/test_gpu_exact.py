@@ -299,6 +299,28 @@ def test_attention_reference_order_nonfinite_v_masked(exact_gpu):
     assert bits_or_nan(got, want)
 
 
+@pytest.mark.parametrize("b,h,sq,sk,d", [(1, 3, 33, 200, 96), (1, 2, 20, 300, 64), (2, 1, 65, 65, 128), (1, 2, 40, 130, 40),
+                                         (8, 33, 130, 64, 64),       # 128 rows a workgroup
+                                         (1, 2, 2, 300, 128)])       # decode
+def test_attention_reference_order_in_place(exact_gpu, b, h, sq, sk, d):
+    """O in Q's place.  V has columns of zeros and an infinite row, so some
+    waves of a workgroup recompute rows on the vector ALUs, which read Q again."""
+    Q = RNG.standard_normal((b, h, sq, d)).astype(np.float32)
+    K = RNG.standard_normal((b, h, sk, d)).astype(np.float32)
+    V = RNG.standard_normal((b, h, sk, d)).astype(np.float32)
+    V[..., d - 3:] = 0.0
+    V[0, 0, sk - 1, 1] = np.inf
+    bq, bk, bv = (exact_gpu.upload(x) for x in (Q, K, V))
+    try:
+        exact_gpu.run(abi.OP_ATTENTION_F32, Q=bq, K=bk, V=bv, O=bq, batch=b, heads=h, seq_q=sq, seq_k=sk, head_dim=d,
+                      causal=1)
+        got = exact_gpu.download(bq, np.float32, Q.shape)
+    finally:
+        for x in (bq, bk, bv):
+            exact_gpu.free(x)
+    assert bits_or_nan(got, block_oracle.attention_threaded(Q, K, V, 1, avx2=True))
+
+
 def test_attention_reference_order_denormal_v(exact_gpu):
     """V of denormal magnitude: products underflow to signed zeros, so the
     sign of a zero accumulator decides the output's bits; the waves with
