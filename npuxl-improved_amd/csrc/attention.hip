@@ -1078,6 +1078,15 @@ size_t attention_ws_bytes(const Attn &a)
     return static_cast<size_t>(splits) * rows * (a.head_dim + 2) * sizeof(float);
 }
 
+const char *attention_route(const Attn &a)
+{
+    return use_exact_tiled(a) ? attention_exact_route(a)
+           : use_rowwise(a)   ? "rowwise"
+           : use_prefill(a)   ? "split_prefill"
+           : use_decode(a)    ? "stream_decode"
+                              : "general";
+}
+
 void attention(hipStream_t s, const Attn &a, float *ws)
 {
     if (use_exact_tiled(a)) {

@@ -56,6 +56,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <type_traits>
 #include "device_math.hpp"
 #include "lds_dma.hpp"
@@ -1062,6 +1063,36 @@ bool aligned16(const Attn &a)
     return true;
 }
 
+// Up to kDecMaxRows rows run as decode or in the 32-row workgroups; the two
+// times, us, fitted to both kernels over 1 to 300 (batch, head) pairs, 1 to 8
+// rows, 8 to 5000 keys and all head sizes (of 1017 calls the rule takes the
+// side that is more than 5% slower for 7; 96 pairs x 4 rows x 4000 keys at
+// head_dim 128 204 against 259, 256 pairs x 4 x 1500 182 against 112).
+//
+// Decode: two launches, K from memory once, and rounds of the chains that fit
+// the chip (two per CU), each longer as they share the CUs.
+double decode_us(const Attn &a)
+{
+    const bool small = a.head_dim <= 64;
+    const double pairs = static_cast<double>(a.batch) * a.heads, cus = cu_count();
+    const double chains = pairs * a.seq_q * ((a.head_dim + 63) / 64);
+    const double load = std::min(1.0, std::max(0.0, (chains / cus - 0.5) / 1.5));
+    const double block = small ? 1.0 + 0.4 * load : 0.95 + 0.6 * load;
+    return (small ? 6.7 : 8.3) + 0.6 * a.seq_q + std::ceil(chains / (2 * cus)) * a.seq_k / XB * block +
+           pairs * a.seq_k * a.head_dim * sizeof(float) * 0.14e-6;
+}
+
+// 32-row workgroups: one for each pair, its blocks in turn; a second one on a
+// CU costs as much again where LDS holds one (head_dim above 64), else half; at
+// the largest head sizes a full chip waits for memory as well.
+double few_rows_us(const Attn &a)
+{
+    const bool small = a.head_dim <= 64;
+    const double fill = static_cast<double>(a.batch) * a.heads / cu_count();
+    const double block = small ? 3.05 : a.head_dim <= 96 ? 4.0 : 4.0 + 0.35 * std::min(1.0, fill);
+    return 3.5 + block * ((a.seq_k + XB - 1) / XB) * (1.0 + (std::ceil(fill) - 1.0) * (small ? 0.55 : 1.0));
+}
+
 }  // namespace
 
 bool attention_exact_supported(const Attn &a)
@@ -1077,20 +1108,14 @@ bool attention_exact_supported(const Attn &a)
 
 bool attention_exact_decodes(const Attn &a)
 {
-    // A row's chains cost two launches and read V once per row; 32-row workgroups
-    // read it once but leave most of their rows idle.  Few keys go to the latter
-    // (32 heads x 4 rows of 40 keys 9.0 -> 6.2 us, 1 row 7.3 -> 6.2), and so do two
-    // to four rows of so many heads that the chains do not fit the chip at once
-    // (256 heads x 4 rows of 160 keys at head_dim 128 40.0 -> 18.2 us).
-    const uint64_t chains = static_cast<uint64_t>(a.batch) * a.heads * a.seq_q * ((a.head_dim + 63) / 64);
     if (a.seq_q <= 4 && !aligned16(a)) return true;   // the chains read Q and write O by dwords
-    if (a.seq_k < std::max(64u, 32 * a.seq_q)) return false;
-    if (a.seq_q <= 4)   // (two rows of a long context: 258 us against 267 for 256 heads x 4000 keys)
-        return a.seq_q == 1 || chains <= 2 * cu_count() || (a.seq_q == 2 && a.seq_k >= 2048);
-    // A few more rows behind a long context (the check of drafted tokens), as
-    // long as the chains fit: 32 heads x 5 rows x 4000 keys at head_dim 128 100 us
-    // against 240 with 32-row workgroups; at 300 keys, or more rows, they lose.
-    return a.seq_q <= kDecMaxRows && a.seq_k >= 1024 && chains <= 2 * cu_count() && dec_scores_bytes(a) <= kDecScoreCap;
+    return a.seq_q <= kDecMaxRows && (a.seq_q <= 4 || dec_scores_bytes(a) <= kDecScoreCap) &&
+           decode_us(a) < few_rows_us(a);
+}
+
+const char *attention_exact_route(const Attn &a)
+{
+    return attention_exact_decodes(a) ? "exact_decode" : share_rows(a) ? "exact_rows32" : "exact_rows128";
 }
 
 void attention_exact_prefill(hipStream_t s, const Attn &a)

@@ -1268,3 +1268,24 @@ void release_device_tables(vnpu_device_t *dev)
 }
 
 }  // namespace vnpu
+
+// What the dispatch rules choose for a command, as text, from its sizes and
+// the alignment of its pointers, none of which is read (a host without a GPU
+// answers for 256 CUs).  For the tests of those rules.
+extern "C" VNPU_API int32_t VNPU_CALL vnpu_debug_route(const vnpu_command_t *cmd, uint32_t high_throughput, char *out,
+                                                       uint32_t size)
+{
+    if (!cmd || !out || !size) return VNPU_ERR_INVALID_ARGUMENT;
+    try {
+        if (cmd->opcode == VNPU_OP_ATTENTION_F32) {
+            const vnpu_attention_f32_args_t &a = cmd->args.attention;
+            vnpu::k::Attn p = vnpu::attention_params(a);
+            p.exact = !high_throughput;
+            p.Q = a.Q; p.K = a.K; p.V = a.V; p.mask = a.mask; p.O = a.O;
+            std::snprintf(out, size, "%s", vnpu::k::attention_route(p));
+            return VNPU_OK;
+        }
+    } catch (...) {
+    }
+    return VNPU_ERR_INVALID_ARGUMENT;
+}

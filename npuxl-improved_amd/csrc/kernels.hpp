@@ -210,12 +210,15 @@ struct Attn {
 };
 size_t attention_ws_bytes(const Attn &a);
 void attention(hipStream_t s, const Attn &a, float *ws);
+// The kernels that the call takes, by name.
+const char *attention_route(const Attn &a);
 // Reference-order attention on the fp32 matrix cores takes the call: head_dim
 // a multiple of 8 up to 128, rows it can copy 16 bytes at a time, and decode
 // scores of one (batch, head) within its workspace cap (attn_exact.hip).
 bool attention_exact_supported(const Attn &a);
-// Whether it runs as decode (up to 4 query rows, and some calls of a few more).
+// Whether it runs as decode (up to 8 query rows, where that is faster).
 bool attention_exact_decodes(const Attn &a);
+const char *attention_exact_route(const Attn &a);
 // Reference-order prefill.
 void attention_exact_prefill(hipStream_t s, const Attn &a);
 // Reference-order decode: scores, then the output chain; ws holds

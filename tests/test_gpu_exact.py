@@ -234,8 +234,9 @@ def test_attention_reference_order_prefill_shapes(exact_gpu, b, h, sq, sk, d, ca
 
 @pytest.mark.parametrize("d", [64, 80, 128])
 @pytest.mark.parametrize("b,h,sq,sk,causal,mask", [
-    (2, 3, 1, 63, 1, None), (2, 3, 1, 64, 0, "normal"),        # one row: 32-row workgroups below 64 keys
-    (1, 2, 4, 127, 0, "inf"), (1, 2, 4, 128, 1, None),         # and four rows below 128
+    (2, 3, 1, 63, 1, None), (2, 3, 1, 64, 0, "normal"), (2, 3, 1, 65, 1, None),   # one row: 32-row workgroups to 64 keys
+    (1, 2, 4, 127, 0, "inf"), (1, 2, 4, 128, 1, None), (1, 2, 4, 129, 0, "normal"),   # and four rows to 128
+    (6, 16, 4, 700, 1, None), (8, 32, 3, 300, 0, None), (3, 16, 8, 200, 1, "normal"),   # 96 and 256 pairs; eight rows
     (1, 3, 2, 12, 1, None), (1, 3, 3, 13, 0, "row"),           # a handful of keys
     (9, 32, 2, 200, 1, None),                                  # rows of many heads
     (2, 33, 1, 2000, 0, None)])                                # scores: two tiles a wave, the last one alone
