@@ -23,6 +23,7 @@
 #include "vnpu_internal.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 
 // Device scratch of vnpu_attention_f32_noalloc (partial (m, l, acc) triples of
@@ -982,16 +983,6 @@ bool use_decode(const Attn &a)
     return a.seq_q <= 4 && (a.head_dim % 32) == 0 && a.head_dim <= 256;
 }
 
-// Reference-order matrix-core kernels.  They also take a high-throughput
-// device's calls that none of its own matrix-core or streaming kernels does
-// (32 heads of 80, 2048 rows: 2580 us with attn_kernel, 332 here; decode of
-// 8 x 32 heads of 80 over 4096 keys: 596 against 138).
-bool use_exact_tiled(const Attn &a)
-{
-    if (use_rowwise(a)) return false;
-    return a.exact || (!use_decode(a) && a.head_dim != 64 && a.head_dim != 128 && attention_exact_supported(a));
-}
-
 bool use_prefill(const Attn &a)
 {
     return !use_decode(a) && (a.head_dim == 64 || a.head_dim == 128);
@@ -1031,6 +1022,37 @@ void plan(const Attn &a, uint32_t &qblocks, uint32_t &splits, uint32_t &kps)
     while (tiles * splits < 2048 && splits * 2 <= kblocks && kblocks / (splits * 2) >= 2) splits *= 2;
     kps = ((kblocks + splits - 1) / splits) * BKEY;
     splits = (a.seq_k + kps - 1) / kps;
+}
+
+// attn_kernel's time, us, fitted over 996 calls (1 to 300 (batch, head) pairs,
+// 1 to 1500 rows, 8 to 5000 keys, head sizes 8 to 120): the blocks of one
+// workgroup in turn, or the CUs' share of them all, and the merge of split keys.
+double general_us(const Attn &a)
+{
+    uint32_t qblocks, splits, kps;
+    plan(a, qblocks, splits, kps);
+    const double d = a.head_dim, bh = static_cast<double>(a.batch) * a.heads, blocks = kps / BKEY;
+    double live = 1.0;   // of the blocks of a whole grid
+    if (a.causal && a.seq_k >= a.seq_q) live = 1.0 - (a.seq_q - std::min<uint32_t>(BQ, a.seq_q)) / (2.0 * a.seq_k);
+    const double share = qblocks * bh * splits * live / cu_count() * blocks;
+    double t = 2.6 + std::hypot(blocks * (8.1 + 0.095 * d), share * (1.1 + 0.091 * d));
+    if (splits > 1) t += 3.1 + 1.05e-6 * sizeof(float) * splits * bh * a.seq_q * d;
+    return t;
+}
+
+// Reference-order matrix-core kernels.  They also take a high-throughput
+// device's calls that none of its own matrix-core or streaming kernels does,
+// where they beat attn_kernel: 32 heads of 80, 2048 rows 2580 -> 332 us, decode of
+// 8 x 32 heads of 80 over 4096 keys 596 -> 138; but few rows or heads behind a
+// long context are a chain of blocks there and split over keys in attn_kernel (8
+// heads of 8, 21 rows, 1986 keys 105 against 27 us; 2 of 112, 21 rows, 2294 keys
+// 166 against 66).  Of the 996 calls of the fit the slower one is taken for five
+// by more than 5% (with the reference-order kernels for all, for 112).
+bool use_exact_tiled(const Attn &a)
+{
+    if (use_rowwise(a)) return false;
+    if (a.exact) return true;
+    return !use_decode(a) && !use_prefill(a) && attention_exact_supported(a) && attention_exact_us(a) < general_us(a);
 }
 
 }  // namespace

@@ -1113,6 +1113,14 @@ bool attention_exact_decodes(const Attn &a)
            decode_us(a) < few_rows_us(a);
 }
 
+double attention_exact_us(const Attn &a)
+{
+    if (attention_exact_decodes(a)) return decode_us(a);
+    // share_rows' estimates, 4.1 and 11.5 us a block at head_dim 128
+    const double tiles = (a.head_dim <= 64 ? 3.05 : 4.0) * std::min(grid_blocks(a, XQW, 1.2), 2.8 * grid_blocks(a, XQ, 0.45));
+    return a.seq_q <= kDecMaxRows ? std::max(tiles, few_rows_us(a)) : tiles;
+}
+
 const char *attention_exact_route(const Attn &a)
 {
     return attention_exact_decodes(a) ? "exact_decode" : share_rows(a) ? "exact_rows32" : "exact_rows128";

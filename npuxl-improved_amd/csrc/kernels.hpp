@@ -218,6 +218,8 @@ const char *attention_route(const Attn &a);
 bool attention_exact_supported(const Attn &a);
 // Whether it runs as decode (up to 8 query rows, where that is faster).
 bool attention_exact_decodes(const Attn &a);
+// Its time, estimated, us.
+double attention_exact_us(const Attn &a);
 const char *attention_exact_route(const Attn &a);
 // Reference-order prefill.
 void attention_exact_prefill(hipStream_t s, const Attn &a);

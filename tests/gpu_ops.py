@@ -10,7 +10,7 @@ import ctypes as C
 
 import numpy as np
 
-from vnpu_mi355x import abi
+from vnpu_mi355x import Session, abi, load_backend
 
 
 def quantize(s, X, axis):
@@ -145,3 +145,14 @@ def mtp_head(s, hidden, W, bias=None, trans_w=0):
         if x is not None:
             s.free(x)
     return out
+
+
+def route(opcode, fast=False, **fields):
+    """What the dispatch rules choose for the call (no GPU needed)."""
+    lib = load_backend()
+    lib.vnpu_debug_route.restype = C.c_int32
+    lib.vnpu_debug_route.argtypes = [C.c_void_p, C.c_uint32, C.c_char_p, C.c_uint32]
+    cmd = Session.command(opcode, **fields)
+    out = C.create_string_buffer(128)
+    assert lib.vnpu_debug_route(C.byref(cmd), int(fast), out, 128) == abi.OK
+    return out.value.decode()

@@ -13,6 +13,7 @@ import pytest
 
 import oracle
 import gpu_ops as g
+from gpu_ops import route
 from vnpu_mi355x import abi
 
 pytestmark = pytest.mark.gpu
@@ -881,6 +882,37 @@ def test_attention(request, dev, b, h, sq, sk, d, causal, use_mask):
     got = g.attention(gpu, Q, K, V, mask, causal)
     want = oracle.attention(Q, K, V, mask, causal)
     assert rel(got, want) <= 2e-3
+
+
+@pytest.mark.parametrize("b,h,sq,sk,d,causal,mask", [
+    # head sizes that only the general kernel takes: one and several values per lane, up to 160 KiB of LDS
+    (1, 3, 40, 40, 160, 0, None), (2, 2, 20, 1000, 192, 1, "normal"), (1, 2, 17, 300, 256, 1, None),
+    (1, 2, 33, 70, 36, 1, "inf"), (1, 1, 3, 2000, 33, 0, "row"), (2, 1, 5, 700, 100, 1, "row"), (1, 2, 1, 65, 1, 1, None),
+    (1, 2, 20, 9, 144, 1, None), (3, 16, 130, 130, 152, 1, "normal"),
+    # and those where it beats the reference-order kernels: the key range split, ragged last blocks and splits
+    (1, 2, 20, 3000, 80, 1, None), (1, 8, 21, 1986, 8, 1, "normal"), (4, 1, 14, 2006, 112, 0, "inf"),
+    (1, 2, 2, 2500, 48, 1, "row")])
+def test_attention_general_kernel(fast_gpu, b, h, sq, sk, d, causal, mask):
+    """attn_kernel and the merge of its split keys.  A weight is the reference's
+    degree-5 polynomial, up to 1.6e-4 off (ln(2)^6 / 720), and the maxima that it
+    is taken against differ from the oracle's where the keys are split: weight,
+    rescale and sum together 5e-4."""
+    assert route(abi.OP_ATTENTION_F32, True, Q=4096, K=4096, V=4096, O=4096, batch=b, heads=h, seq_q=sq, seq_k=sk,
+                 head_dim=d, causal=causal) == "general"
+    Q = RNG.standard_normal((b, h, sq, d)).astype(np.float32)
+    K = RNG.standard_normal((b, h, sk, d)).astype(np.float32)
+    V = RNG.standard_normal((b, h, sk, d)).astype(np.float32)
+    M = None
+    if mask:
+        M = RNG.standard_normal((b, h, sq, sk)).astype(np.float32)
+        if mask == "inf":
+            M[..., sk // 4:sk // 2] = -np.inf              # whole splits without a key
+        if mask == "row":
+            M[:, 0, 0, :] = -np.inf
+    got = g.attention(fast_gpu, Q, K, V, M, causal)
+    assert rel(got, oracle.attention(Q, K, V, M, causal)) <= 5e-4
+    if mask == "row":
+        assert not got[:, 0, 0].any()
 
 
 @pytest.mark.parametrize("b,h,sq,sk,d,causal", [

@@ -2,21 +2,10 @@
 256 CUs).  Each row is a call whose two sides were timed on an MI355X: the
 route is the faster one.
 """
-import ctypes as C
-
 import pytest
 
-from vnpu_mi355x import Session, abi, load_backend
-
-
-def route(opcode, fast=False, **fields):
-    lib = load_backend()
-    lib.vnpu_debug_route.restype = C.c_int32
-    lib.vnpu_debug_route.argtypes = [C.c_void_p, C.c_uint32, C.c_char_p, C.c_uint32]
-    cmd = Session.command(opcode, **fields)
-    out = C.create_string_buffer(128)
-    assert lib.vnpu_debug_route(C.byref(cmd), int(fast), out, 128) == abi.OK
-    return out.value.decode()
+from gpu_ops import route
+from vnpu_mi355x import abi
 
 
 def attention(pairs, sq, sk, d, fast=False, causal=1, off=0):
@@ -47,3 +36,21 @@ def test_attention_few_rows_unaligned():
     """Rows that are not 16-byte aligned: the chains at head sizes 64 and 128, else the row-wise kernel."""
     assert attention(256, 4, 300, 128, off=4) == "exact_decode"
     assert attention(256, 4, 300, 96, off=4) == "rowwise"
+
+
+@pytest.mark.parametrize("pairs,sq,sk,d,want", [
+    # high-throughput device, head sizes without a kernel of its own: general against reference-order, us
+    (8, 21, 1986, 8, "general"),            # 27 / 105
+    (4, 67, 3819, 24, "general"),           # 54 / 184
+    (4, 14, 2006, 80, "general"),           # 43 / 122
+    (2, 21, 2294, 112, "general"),          # 66 / 166
+    (64, 7, 974, 24, "general"),            # 30 / 51
+    (32, 2048, 2048, 80, "exact_rows128"),  # 2580 / 332
+    (256, 1, 4096, 80, "exact_decode"),     # 596 / 138
+    (32, 64, 99, 72, "exact_rows32"),       # 35 / 13
+    (32, 333, 1501, 96, "exact_rows32"),
+    # its own kernels keep theirs
+    (8, 21, 1986, 64, "split_prefill"), (32, 1, 4096, 128, "stream_decode"), (32, 4, 300, 96, "stream_decode"),
+    (4, 20, 300, 160, "general"), (4, 20, 300, 36, "general"), (4, 20, 300, 300, "rowwise")])
+def test_attention_high_throughput(pairs, sq, sk, d, want):
+    assert attention(pairs, sq, sk, d, fast=True) == want
