@@ -778,7 +778,7 @@ VNPU_API vnpu_status_t VNPU_CALL vnpu_pack_weights_i8_masked(vnpu_device_t *devi
 
 /* MI355X extension (additive; no counterpart in the reference): ATTENTION_F32
  * that allocates nothing, for callers that cannot allocate device memory
- * (code under HIP graph capture, serving loops).  Same arguments and kernels
+ * (code under HIP graph capture, serving loops).  Same arguments and output
  * as vnpu_attention_f32, but Q, K, V, mask and O must be device memory
  * (vnpu_buffer_host_ptr or hipMalloc), the call only enqueues on the stream
  * (completion: vnpu_stream_sync or later work on the stream), and its
@@ -786,7 +786,8 @@ VNPU_API vnpu_status_t VNPU_CALL vnpu_pack_weights_i8_masked(vnpu_device_t *devi
  * process: shapes needing more (the split K/V^T blocks of prefill beyond
  * 64 MiB, e.g. 32 heads x more than 2048 keys at head_dim 128) return
  * VNPU_ERR_INVALID_ARGUMENT, as do host pointers.  Every call on a GPU shares
- * that array, so calls that overlap on one GPU race. */
+ * that array, so calls that overlap on one GPU race.  (On a default device
+ * only up to 4 query rows at head_dim 64 and 128 use it.) */
 VNPU_API vnpu_status_t VNPU_CALL vnpu_attention_f32_noalloc(vnpu_stream_t *stream,
                                                             const vnpu_attention_f32_args_t *args);
 

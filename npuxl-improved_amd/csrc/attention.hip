@@ -1052,7 +1052,10 @@ bool use_exact_tiled(const Attn &a)
 {
     if (use_rowwise(a)) return false;
     if (a.exact) return true;
-    return !use_decode(a) && !use_prefill(a) && attention_exact_supported(a) && attention_exact_us(a) < general_us(a);
+    if (use_decode(a) || use_prefill(a) || !attention_exact_supported(a)) return false;
+    Attn own = a;   // one choice, so one output, whoever owns the workspace
+    own.own_ws = true;
+    return attention_exact_us(own) < general_us(a);
 }
 
 }  // namespace

@@ -1109,6 +1109,9 @@ bool attention_exact_supported(const Attn &a)
 bool attention_exact_decodes(const Attn &a)
 {
     if (a.seq_q <= 4 && !aligned16(a)) return true;   // the chains read Q and write O by dwords
+    // Where the workspace is shared with calls on other streams, which race for
+    // it, only the rows that have always taken it do (the output is the same).
+    if (!a.own_ws && !(a.seq_q <= 4 && (a.head_dim == 64 || a.head_dim == 128))) return false;
     return a.seq_q <= kDecMaxRows && (a.seq_q <= 4 || dec_scores_bytes(a) <= kDecScoreCap) &&
            decode_us(a) < few_rows_us(a);
 }

@@ -1058,6 +1058,7 @@ void enqueue_attention_noalloc(vnpu_stream_t *s, const vnpu_attention_f32_args_t
                 is_device_pointer(a.O) && (!a.mask || is_device_pointer(a.mask)),
             "attention without allocation needs device-resident Q, K, V, mask and O");
     p.Q = a.Q; p.K = a.K; p.V = a.V; p.mask = a.mask; p.O = a.O;
+    p.own_ws = false;
     const size_t need = k::attention_ws_bytes(p);
     if (need > k::kAttnScratchBytes) {
         debug_log("attention without allocation: this call needs %zu bytes of scratch, above the "
@@ -1271,8 +1272,9 @@ void release_device_tables(vnpu_device_t *dev)
 
 // What the dispatch rules choose for a command, as text, from its sizes and
 // the alignment of its pointers, none of which is read (a host without a GPU
-// answers for 256 CUs).  For the tests of those rules.
-extern "C" VNPU_API int32_t VNPU_CALL vnpu_debug_route(const vnpu_command_t *cmd, uint32_t high_throughput, char *out,
+// answers for 256 CUs).  mode: 1 a high-throughput device, 2 an attention call
+// on the shared scratch.  For the tests of those rules.
+extern "C" VNPU_API int32_t VNPU_CALL vnpu_debug_route(const vnpu_command_t *cmd, uint32_t mode, char *out,
                                                        uint32_t size)
 {
     if (!cmd || !out || !size) return VNPU_ERR_INVALID_ARGUMENT;
@@ -1280,9 +1282,10 @@ extern "C" VNPU_API int32_t VNPU_CALL vnpu_debug_route(const vnpu_command_t *cmd
         if (cmd->opcode == VNPU_OP_ATTENTION_F32) {
             const vnpu_attention_f32_args_t &a = cmd->args.attention;
             vnpu::k::Attn p = vnpu::attention_params(a);
-            p.exact = !high_throughput;
+            p.exact = !(mode & 1u);
+            p.own_ws = !(mode & 2u);
             p.Q = a.Q; p.K = a.K; p.V = a.V; p.mask = a.mask; p.O = a.O;
-            std::snprintf(out, size, "%s", vnpu::k::attention_route(p));
+            std::snprintf(out, size, "%s ws=%zu", vnpu::k::attention_route(p), vnpu::k::attention_ws_bytes(p));
             return VNPU_OK;
         }
     } catch (...) {

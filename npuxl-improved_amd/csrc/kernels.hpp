@@ -207,6 +207,7 @@ struct Attn {
     uint32_t batch = 0, heads = 0, seq_q = 0, seq_k = 0, head_dim = 0, causal = 0;
     float scale = 1.0f;
     bool exact = false;   // the reference's order of roundings (bit for bit)
+    bool own_ws = true;   // the workspace is this call's: else take none where none is needed
 };
 size_t attention_ws_bytes(const Attn &a);
 void attention(hipStream_t s, const Attn &a, float *ws);

@@ -774,7 +774,8 @@ VNPU_API void *VNPU_CALL vnpu_stream_hip_handle(vnpu_stream_t *stream)
 
 // ATTENTION_F32 that allocates nothing (no reference counterpart): for
 // callers that cannot allocate device memory, such as code under HIP graph
-// capture or a serving loop.  The kernels are vnpu_attention_f32's; their
+// capture or a serving loop.  The output is vnpu_attention_f32's, from kernels
+// that need no scratch where there are such; else the
 // scratch is the per-GPU device array of attention.hip (set up by
 // vnpu_device_create), shared by every call on that GPU, so calls that
 // overlap on one GPU (two streams, two threads) race.  Enqueues only.

@@ -147,12 +147,12 @@ def mtp_head(s, hidden, W, bias=None, trans_w=0):
     return out
 
 
-def route(opcode, fast=False, **fields):
+def route(opcode, fast=False, noalloc=False, **fields):
     """What the dispatch rules choose for the call (no GPU needed)."""
     lib = load_backend()
     lib.vnpu_debug_route.restype = C.c_int32
     lib.vnpu_debug_route.argtypes = [C.c_void_p, C.c_uint32, C.c_char_p, C.c_uint32]
     cmd = Session.command(opcode, **fields)
     out = C.create_string_buffer(128)
-    assert lib.vnpu_debug_route(C.byref(cmd), int(fast), out, 128) == abi.OK
+    assert lib.vnpu_debug_route(C.byref(cmd), int(fast) + 2 * int(noalloc), out, 128) == abi.OK
     return out.value.decode()

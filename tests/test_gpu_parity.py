@@ -898,7 +898,7 @@ def test_attention_general_kernel(fast_gpu, b, h, sq, sk, d, causal, mask):
     is taken against differ from the oracle's where the keys are split: weight,
     rescale and sum together 5e-4."""
     assert route(abi.OP_ATTENTION_F32, True, Q=4096, K=4096, V=4096, O=4096, batch=b, heads=h, seq_q=sq, seq_k=sk,
-                 head_dim=d, causal=causal) == "general"
+                 head_dim=d, causal=causal).startswith("general")
     Q = RNG.standard_normal((b, h, sq, d)).astype(np.float32)
     K = RNG.standard_normal((b, h, sk, d)).astype(np.float32)
     V = RNG.standard_normal((b, h, sk, d)).astype(np.float32)

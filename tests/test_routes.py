@@ -8,10 +8,12 @@ from gpu_ops import route
 from vnpu_mi355x import abi
 
 
-def attention(pairs, sq, sk, d, fast=False, causal=1, off=0):
+def attention(pairs, sq, sk, d, fast=False, causal=1, off=0, noalloc=False):
+    """(kernels, bytes of workspace)"""
     p = [4096 * (i + 1) + off for i in range(4)]
-    return route(abi.OP_ATTENTION_F32, fast, Q=p[0], K=p[1], V=p[2], O=p[3], batch=1, heads=pairs, seq_q=sq, seq_k=sk,
-                 head_dim=d, causal=causal)
+    name, ws = route(abi.OP_ATTENTION_F32, fast, noalloc, Q=p[0], K=p[1], V=p[2], O=p[3], batch=1, heads=pairs,
+                     seq_q=sq, seq_k=sk, head_dim=d, causal=causal).split(" ws=")
+    return name, int(ws)
 
 
 @pytest.mark.parametrize("pairs,sq,sk,d,want", [
@@ -29,13 +31,13 @@ def attention(pairs, sq, sk, d, fast=False, causal=1, off=0):
     (8, 1, 4000, 128, "exact_decode"), (8, 2, 64, 128, "exact_rows32"), (8, 8, 4000, 64, "exact_decode"),
     (8, 9, 4000, 64, "exact_rows32"), (32, 2048, 2048, 128, "exact_rows128")])
 def test_attention_few_rows(pairs, sq, sk, d, want):
-    assert attention(pairs, sq, sk, d) == want
+    assert attention(pairs, sq, sk, d)[0] == want
 
 
 def test_attention_few_rows_unaligned():
     """Rows that are not 16-byte aligned: the chains at head sizes 64 and 128, else the row-wise kernel."""
-    assert attention(256, 4, 300, 128, off=4) == "exact_decode"
-    assert attention(256, 4, 300, 96, off=4) == "rowwise"
+    assert attention(256, 4, 300, 128, off=4)[0] == "exact_decode"
+    assert attention(256, 4, 300, 96, off=4)[0] == "rowwise"
 
 
 @pytest.mark.parametrize("pairs,sq,sk,d,want", [
@@ -53,4 +55,16 @@ def test_attention_few_rows_unaligned():
     (8, 21, 1986, 64, "split_prefill"), (32, 1, 4096, 128, "stream_decode"), (32, 4, 300, 96, "stream_decode"),
     (4, 20, 300, 160, "general"), (4, 20, 300, 36, "general"), (4, 20, 300, 300, "rowwise")])
 def test_attention_high_throughput(pairs, sq, sk, d, want):
-    assert attention(pairs, sq, sk, d, fast=True) == want
+    assert attention(pairs, sq, sk, d, fast=True)[0] == want
+
+
+@pytest.mark.parametrize("pairs,sq,sk,d", [(96, 1, 4000, 96), (64, 6, 4000, 64), (8, 5, 2000, 128), (8, 4, 4000, 80)])
+def test_attention_shared_scratch(pairs, sq, sk, d):
+    """On the scratch that all streams share, calls that can do without it do."""
+    assert attention(pairs, sq, sk, d)[0] == "exact_decode"
+    assert attention(pairs, sq, sk, d, noalloc=True) == ("exact_rows32", 0)
+    assert attention(pairs, sq, sk, 8, fast=True, noalloc=True)[0] == attention(pairs, sq, sk, 8, fast=True)[0]
+
+
+def test_attention_shared_scratch_decode():
+    assert attention(32, 1, 4000, 128, noalloc=True) == attention(32, 1, 4000, 128) == ("exact_decode", 32 * 4032 * 4)

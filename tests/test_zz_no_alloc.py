@@ -1,8 +1,8 @@
 """vnpu_attention_f32_noalloc: ATTENTION_F32 with the per-GPU device scratch.
 
 Through the C ABI, on device-resident tensors: two calls in a row, the
-second with a smaller input, each compared with vnpu_attention_f32 (the
-same kernels with the stream workspace) bit for bit and with the C oracle
+second with a smaller input, each compared with vnpu_attention_f32 (which
+takes its workspace from the stream) bit for bit and with the C oracle
 within the attention bar; shapes above the 64 MiB scratch and host pointers
 are refused without running anything.
 """
@@ -65,6 +65,11 @@ def _case(gpu, b, h, sq, sk, d, causal, use_mask):
     # default device, reference-order decode (the scores in the scratch):
     # config-4 decode, then three query rows at head_dim 64 with a mask
     ("gpu", (8, 32, 1, 4096, 128, 1, False), (2, 4, 3, 1000, 64, 1, True)),
+    # default device, decode that runs without the scratch here: one row at
+    # head_dim 96, then six rows at 64 behind a long context
+    ("gpu", (6, 16, 1, 2000, 96, 1, False), (4, 16, 6, 1500, 64, 1, True)),
+    # the general kernel at head sizes that only it takes, key ranges split
+    ("fast_gpu", (1, 2, 20, 3000, 160, 1, False), (1, 1, 5, 700, 36, 0, True)),
 ])
 def test_noalloc_matches_attention_two_calls(request, dev, first, second):
     gpu = request.getfixturevalue(dev)
