@@ -47,6 +47,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdio>
 
 namespace vnpu {
 namespace k {
@@ -65,9 +66,9 @@ constexpr int kNontemporal = 2;           // cache policy bits
 // without spills (18.8 -> 22.9 us at 256 x 4096 x 4096).
 template <int MG, int W, bool SHIFT>
 constexpr int kWavesPerSimd = MG == 4 ? 1 : MG == 2 && W == 4 ? 3 : MG == 2 && !SHIFT ? 2 : 4;
-template <int MG, int CB, int W, bool SHIFT, bool STREAM>
+template <int MG, int CB, int W, bool SHIFT, bool STREAM, bool SPREAD>
 __global__ __launch_bounds__(64 * W)
-__attribute__((amdgpu_waves_per_eu(kWavesPerSimd<MG, W, SHIFT>))) void direct_i8_kernel(I8Gemm p)
+__attribute__((amdgpu_waves_per_eu(kWavesPerSimd<MG, W, SHIFT>))) void direct_i8_kernel(I8Gemm p, uint32_t last)
 {
     constexpr int TILE = 256 * MG * CB;                       // sums of a wave
     constexpr int S = 16384 / TILE < W ? 16384 / TILE : W;    // waves' sums in LDS at a time (64 KiB)
@@ -79,8 +80,19 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<MG, W, SHIFT>))) void direct_i8
     // Workgroups are dealt to the eight XCDs in turn: the row tiles of a column
     // tile are neighbours on one, so its L2 fetches the weights once (with the
     // row tiles a whole pass over the columns apart 331 x 1376 x 5003 took 22.5
-    // instead of 17.8 us, 48 x 4096 x 32000 61 instead of 45).
-    const uint32_t nt0 = (blockIdx.y * 8 + (blockIdx.x & 7u)) * CB, m0 = (blockIdx.x >> 3) * (16 * MG);
+    // instead of 17.8 us, 48 x 4096 x 32000 61 instead of 45).  The column tiles
+    // go to the XCDs in turn too; with SPREAD the tiles of the last, less than
+    // eight, are dealt out evenly, `last` to each XCD.
+    uint32_t nt0 = (blockIdx.y * 8 + (blockIdx.x & 7u)) * CB, m0 = (blockIdx.x >> 3) * (16 * MG);
+    if constexpr (SPREAD) {
+        if (blockIdx.y + 1 == gridDim.y) {
+            const uint32_t row_tiles = gridDim.x >> 3, i = blockIdx.x >> 3;
+            if (i >= last) return;
+            const uint32_t tile = (blockIdx.x & 7u) * last + i;
+            nt0 = (blockIdx.y * 8 + tile / row_tiles) * CB;
+            m0 = tile % row_tiles * (16 * MG);
+        }
+    }
     if (nt0 >= NT) return;
     const uint32_t rows = min(16u * MG, p.M - m0);
 
@@ -196,8 +208,8 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<MG, W, SHIFT>))) void direct_i8
 }
 
 // Workgroup shapes: 16 mg rows x 16 cb columns, `waves` waves.  The time of a call
-// is start + rounds (round + per_kib K / 1024), us, with rounds = workgroups / CUs
-// rounded up; fitted to the shapes' sweeps over 16..1024 rows at the sizes above
+// is start + rounds (round + per_kib K / 1024), us, with rounds = the workgroups of
+// an XCD / its CUs, rounded up; fitted to the shapes' sweeps over 16..1024 rows at the sizes above
 // (they miss by some 15% at most where they are chosen).  Few rows want narrow
 // workgroups on every CU, more rows larger ones that load less per product; four
 // waves instead of eight let a CU hold more workgroups.  odd_round: `round` for
@@ -234,6 +246,26 @@ bool streams(const I8Gemm &p, uint32_t tile_rows)
 
 bool odd_rows(const I8Gemm &p) { return p.lda % 4 || reinterpret_cast<uintptr_t>(p.A) % 4; }
 
+// The most tiles that an XCD gets, `last` of them from the column tiles past the
+// last whole eight.  Of 9 column tiles in turn one XCD gets two, and of 2 six XCDs
+// get none: their tiles are spread where that saves a round of workgroups (331 x
+// 4096 x 576 11.4 -> 7.6 us, 781 x 8320 x 1088 46.4 -> 26.0, 2048 x 4096 x 128 21.2 ->
+// 8.0).  Elsewhere it would only have more XCDs read their weights (256 x 11008 x 576
+// 13.8 against 14.6 us) and a workgroup wait for one more argument (0.2 us).
+struct Grid {
+    uint64_t tiles;
+    uint32_t xcd_tiles, last;
+    bool spread;
+};
+Grid grid_of(const I8Gemm &p, uint32_t mg, uint32_t cb)
+{
+    const uint64_t cols = (p.Np / 16 + cb - 1) / cb, row_tiles = (p.M + 16 * mg - 1) / (16 * mg);
+    const uint64_t last = (cols % 8 * row_tiles + 7) / 8, even = cols / 8 * row_tiles + last;
+    const uint64_t in_turn = (cols + 7) / 8 * row_tiles, cus = std::max(1u, cu_count() / 8);
+    const bool spread = !streams(p, 16 * mg) && (in_turn + cus - 1) / cus > (even + cus - 1) / cus;
+    return {cols * row_tiles, static_cast<uint32_t>(spread ? even : in_turn), static_cast<uint32_t>(last), spread};
+}
+
 // The shape that should finish first, and its time.
 const Shape &choose(const I8Gemm &p, double &best)
 {
@@ -243,8 +275,9 @@ const Shape &choose(const I8Gemm &p, double &best)
     for (const Shape &h : kShapes) {
         if ((odd && h.odd_round == 0.0) || (h.mg > 1 && p.M <= 8 * h.mg)) continue;
         const uint32_t rows = 16 * h.mg;
-        const uint64_t cols = (p.Np / 16 + h.cb - 1) / h.cb, wgs = cols * ((p.M + rows - 1) / rows);
-        const uint64_t rounds = (wgs + cus - 1) / cus;
+        const Grid g = grid_of(p, h.mg, h.cb);
+        const uint64_t cols = (p.Np / 16 + h.cb - 1) / h.cb, wgs = g.tiles;
+        const uint64_t rounds = (8ull * g.xcd_tiles + cus - 1) / cus;
         // memory and the CUs' own pace overlap, but not wholly where they are alike;
         // a last round that is part empty leaves bandwidth unused as well
         const double fill = rounds > 1 ? std::sqrt(static_cast<double>(wgs) / (rounds * cus)) : 1.0;
@@ -262,17 +295,21 @@ template <int MG, int CB, int W, bool UNALIGNED>
 void launch(hipStream_t s, const I8Gemm &p)
 {
     const uint32_t row_tiles = (p.M + 16 * MG - 1) / (16 * MG);
+    const Grid g = grid_of(p, MG, CB);
     const dim3 grid(8 * row_tiles, (p.Np / 16 + 8 * CB - 1) / (8 * CB));
     if constexpr (UNALIGNED) {
         if (odd_rows(p)) {
-            direct_i8_kernel<MG, CB, W, true, false><<<grid, 64 * W, 0, s>>>(p);
+            if (g.spread) direct_i8_kernel<MG, CB, W, true, false, true><<<grid, 64 * W, 0, s>>>(p, g.last);
+            else direct_i8_kernel<MG, CB, W, true, false, false><<<grid, 64 * W, 0, s>>>(p, 0);
             return;
         }
     }
     if (streams(p, 16 * MG))
-        direct_i8_kernel<MG, CB, W, false, true><<<grid, 64 * W, 0, s>>>(p);
+        direct_i8_kernel<MG, CB, W, false, true, false><<<grid, 64 * W, 0, s>>>(p, 0);
+    else if (g.spread)
+        direct_i8_kernel<MG, CB, W, false, false, true><<<grid, 64 * W, 0, s>>>(p, g.last);
     else
-        direct_i8_kernel<MG, CB, W, false, false><<<grid, 64 * W, 0, s>>>(p);
+        direct_i8_kernel<MG, CB, W, false, false, false><<<grid, 64 * W, 0, s>>>(p, 0);
 }
 
 }  // namespace
@@ -303,6 +340,16 @@ bool direct_i8_takes(const I8Gemm &p)
     double direct;
     choose(p, direct);
     return direct * 1.1 < staged;
+}
+
+void direct_i8_route(const I8Gemm &p, char *out, size_t size)
+{
+    double t;
+    const Shape &h = choose(p, t);
+    const Grid g = grid_of(p, h.mg, h.cb);
+    std::snprintf(out, size, "direct<%u,%u,%u%s%s> tiles=%llu xcd_tiles=%u", h.mg, h.cb, h.waves,
+                  odd_rows(p) ? ",shift" : streams(p, 16 * h.mg) ? ",stream" : "", g.spread ? ",spread" : "",
+                  static_cast<unsigned long long>(g.tiles), g.xcd_tiles);
 }
 
 void direct_i8(hipStream_t s, const I8Gemm &p)

@@ -1288,6 +1288,20 @@ extern "C" VNPU_API int32_t VNPU_CALL vnpu_debug_route(const vnpu_command_t *cmd
             std::snprintf(out, size, "%s ws=%zu", vnpu::k::attention_route(p), vnpu::k::attention_ws_bytes(p));
             return VNPU_OK;
         }
+        if (cmd->opcode == VNPU_OP_MATMUL_I8) {   // dense weights
+            const vnpu_matmul_i8_args_t &a = cmd->args.matmul_i8;
+            if (!a.M || !a.N || !a.K) return VNPU_ERR_INVALID_ARGUMENT;
+            vnpu::k::I8Gemm p;
+            p.M = a.M; p.N = a.N; p.K = a.K;
+            p.lda = a.lda ? a.lda : a.K;
+            p.ldc = a.ldc ? a.ldc : a.N;
+            p.Kp = vnpu::cdiv(a.K, 64u) * 64;
+            p.Np = vnpu::cdiv(a.N, 16u) * 16;
+            p.A = a.A;
+            if (vnpu::k::direct_i8_takes(p)) vnpu::k::direct_i8_route(p, out, size);
+            else std::snprintf(out, size, "%s", a.M <= vnpu::k::kGemvMaxRows ? "gemv" : "gemm");
+            return VNPU_OK;
+        }
     } catch (...) {
     }
     return VNPU_ERR_INVALID_ARGUMENT;

@@ -87,6 +87,8 @@ void gemv_i8(hipStream_t s, const I8Gemm &p);
 // weights (direct_i8.hip): the call is faster there than on gemv_i8 and gemm_i8.
 bool direct_i8_takes(const I8Gemm &p);
 void direct_i8(hipStream_t s, const I8Gemm &p);
+// Its instance (rows and columns / 16, waves), tiles and tiles of an XCD, by name.
+void direct_i8_route(const I8Gemm &p, char *out, size_t size);
 // Any M, int8 MFMA; ws holds gemm_i8_ws_bytes(p) (the strip kernel's A in
 // fragment blocks; nothing for the dense kernels, where ws may be null).
 size_t gemm_i8_ws_bytes(const I8Gemm &p);

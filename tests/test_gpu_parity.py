@@ -327,7 +327,7 @@ def test_matmul_i8_few_rows(gpu, M, K, N):
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
-@pytest.mark.parametrize("M,K,N,lda_pad,off,ldc_pad", [
+DIRECT_I8 = [  # M, K, N, lda - K, bytes before A, ldc - N
     # every workgroup shape (16 x 16 to 64 x 64), whole and with a row, a column or a depth over
     (16, 4096, 4096, 0, 0, 0), (32, 4096, 4096, 0, 0, 0), (64, 4096, 4096, 0, 0, 0), (96, 4096, 4096, 0, 0, 0),
     (200, 4096, 4096, 0, 0, 0), (200, 1024, 2000, 0, 0, 5), (331, 1376, 5003, 0, 0, 0), (65, 4160, 4111, 0, 0, 0),
@@ -339,7 +339,16 @@ def test_matmul_i8_few_rows(gpu, M, K, N):
     (9, 1, 1, 0, 0, 0), (64, 3, 5, 0, 1, 0), (100, 64, 16, 0, 4, 0), (11, 200, 40, 0, 0, 0),
     # weights past the last-level cache, one row tile; five to eight rows of wide weights
     (5, 1000, 16400, 0, 0, 0), (8, 4096, 24700, 0, 0, 0), (7, 333, 20001, 0, 1, 2), (28, 4096, 24700, 0, 0, 0),
-    (60, 4160, 24577, 0, 0, 0)])
+    (60, 4160, 24577, 0, 0, 0),
+    # tiles of the last column tiles spread over the XCDs, each shape
+    (517, 576, 19, 0, 0, 0), (672, 602, 18, 0, 1, 0), (564, 128, 16, 0, 0, 3), (733, 239, 17, 2, 0, 0),
+    (1455, 88, 67, 0, 0, 0), (1584, 1369, 87, 0, 0, 0), (1204, 72, 805, 0, 0, 0), (1638, 75, 156, 1, 0, 0),
+    (1163, 66, 17, 1, 0, 1), (646, 3776, 1343, 0, 0, 0),
+    # instances that none of the above takes
+    (10, 576, 18, 0, 0, 0), (21, 1692, 4139, 1, 0, 0), (9, 5256, 19030, 0, 0, 0), (17, 2176, 47069, 0, 0, 0)]
+
+
+@pytest.mark.parametrize("M,K,N,lda_pad,off,ldc_pad", DIRECT_I8)
 def test_matmul_i8_direct(gpu, M, K, N, lda_pad, off, ldc_pad):
     """Rows between the GEMV and the staged tiles, and rows of any alignment
     (direct_i8.hip): bit-exact against the float64 accumulator, which is the exact

@@ -2,9 +2,12 @@
 256 CUs).  Each row is a call whose two sides were timed on an MI355X: the
 route is the faster one.
 """
+import re
+
 import pytest
 
 from gpu_ops import route
+from test_gpu_parity import DIRECT_I8
 from vnpu_mi355x import abi
 
 
@@ -68,3 +71,31 @@ def test_attention_shared_scratch(pairs, sq, sk, d):
 
 def test_attention_shared_scratch_decode():
     assert attention(32, 1, 4000, 128, noalloc=True) == attention(32, 1, 4000, 128) == ("exact_decode", 32 * 4032 * 4)
+
+
+@pytest.mark.parametrize("M,K,N", [(331, 4096, 576), (1024, 4096, 256), (781, 8320, 1088), (331, 1376, 5003), (9, 64, 16),
+                                   (96, 4096, 1152), (40, 4096, 4111), (2048, 1001, 300)])
+def test_matmul_i8_tiles_of_an_xcd(M, K, N):
+    """The direct kernel's tiles take no more rounds on any XCD than spread evenly over the eight
+    (whole column tiles to the XCDs in turn gave 42 of 168 to one of them for 331 x 4096 x 576)."""
+    name, tiles, per = re.fullmatch(r"direct<(.*)> tiles=(\d+) xcd_tiles=(\d+)",
+                                    route(abi.OP_MATMUL_I8, A=4096, M=M, K=K, N=N)).groups()
+    mg, cb = (int(x) for x in name.split(",")[:2])
+    assert int(tiles) == -(-M // (16 * mg)) * -(-N // (16 * cb))
+    assert int(tiles) <= 8 * int(per)
+    assert -(-int(per) // 32) == -(-int(tiles) // 256)
+
+
+def test_matmul_i8_direct_instances():
+    """The direct kernel's GPU test runs every instance that is built (but the 16 x 16 tiles of weights
+    past the last-level cache, which take a depth beyond 400,000)."""
+    seen = set()
+    for M, K, N, pad, off, _ in DIRECT_I8:
+        t = route(abi.OP_MATMUL_I8, A=4096 + off, M=M, K=K, N=N, lda=K + pad)
+        if t.startswith("direct"):
+            seen.add(t.split()[0])
+    narrow = ("1,1,16", "1,2,8", "1,4,8", "2,4,8")
+    want = {f"direct<{i}{o}>" for i in narrow for o in ("", ",spread", ",shift", ",shift,spread", ",stream")}
+    want.remove("direct<1,1,16,stream>")
+    want |= {f"direct<{i}{o}>" for i in ("2,4,4", "4,4,4") for o in ("", ",spread", ",stream")}
+    assert seen == want
