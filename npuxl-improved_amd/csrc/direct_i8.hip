@@ -70,9 +70,9 @@ template <int MG, int CB, int W, bool SHIFT, bool STREAM, bool SPREAD>
 __global__ __launch_bounds__(64 * W)
 __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<MG, W, SHIFT>))) void direct_i8_kernel(I8Gemm p, uint32_t last)
 {
-    constexpr int TILE = 256 * MG * CB;                       // sums of a wave
-    constexpr int S = 16384 / TILE < W ? 16384 / TILE : W;    // waves' sums in LDS at a time (64 KiB)
-    __shared__ int red[S][16 * MG][16 * CB];
+    constexpr int TILE = 256 * MG * CB;   // sums of a wave
+    static_assert(W * TILE <= 16384, "the waves' sums take 64 KiB of LDS at most");
+    __shared__ int red[W][16 * MG][16 * CB];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, c = lane & 15;
@@ -169,38 +169,20 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<MG, W, SHIFT>))) void direct_i8
         multiply(y);
     }
 
-    // acc[m][b][i]: row 16m + 4g + i, column 16b + c.  S waves at a time hand
-    // their sums to the first S.
-    auto write = [&](int slot) {
+    // acc[m][b][i]: row 16m + 4g + i, column 16b + c.
 #pragma unroll
-        for (int m = 0; m < MG; ++m)
+    for (int m = 0; m < MG; ++m)
 #pragma unroll
-            for (int b = 0; b < CB; ++b)
+        for (int b = 0; b < CB; ++b)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) red[slot][16 * m + 4 * g + i][16 * b + c] = acc[m][b][i];
-    };
-#pragma unroll
-    for (int w0 = W - S; w0 > 0; w0 -= S) {
-        if (wave >= w0 && wave < w0 + S) write(wave - w0);
-        __syncthreads();
-        if (wave < S) {
-#pragma unroll
-            for (int m = 0; m < MG; ++m)
-#pragma unroll
-                for (int b = 0; b < CB; ++b)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) acc[m][b][i] += red[wave][16 * m + 4 * g + i][16 * b + c];
-        }
-        __syncthreads();
-    }
-    if (wave < S) write(wave);
+            for (int i = 0; i < 4; ++i) red[wave][16 * m + 4 * g + i][16 * b + c] = acc[m][b][i];
     __syncthreads();
     for (int o = tid; o < TILE; o += 64 * W) {
         const uint32_t m = m0 + o / (16 * CB), n = nt0 * 16 + o % (16 * CB);
         if (m >= p.M || n >= p.N) continue;
         int v = 0;
 #pragma unroll
-        for (int s = 0; s < S; ++s) v += red[s][o / (16 * CB)][o % (16 * CB)];
+        for (int w = 0; w < W; ++w) v += red[w][o / (16 * CB)][o % (16 * CB)];
         float out = dev::mul_rn(dev::mul_rn(static_cast<float>(v), p.scale_a ? p.scale_a[m] : 1.0f), p.scale_b[n]);
         if (p.bias) out = dev::add_rn(out, p.bias[n]);
         p.C[static_cast<uint64_t>(m) * p.ldc + n] = dev::epilogue(out, p.epilogue);
