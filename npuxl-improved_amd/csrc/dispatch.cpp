@@ -1288,6 +1288,23 @@ extern "C" VNPU_API int32_t VNPU_CALL vnpu_debug_route(const vnpu_command_t *cmd
             std::snprintf(out, size, "%s ws=%zu", vnpu::k::attention_route(p), vnpu::k::attention_ws_bytes(p));
             return VNPU_OK;
         }
+        if (cmd->opcode == VNPU_OP_MATMUL_F32) {   // no tile mask, no requested K depth
+            const vnpu_matmul_f32_args_t &a = cmd->args.matmul_f32;
+            if (!a.M || !a.N || !a.K) return VNPU_ERR_INVALID_ARGUMENT;
+            vnpu::k::F32Gemm p;
+            p.M = a.M; p.N = a.N; p.K = a.K;
+            p.lda = a.lda ? a.lda : (a.trans_a ? a.M : a.K);
+            p.ldb = a.ldb ? a.ldb : (a.trans_b ? a.K : a.N);
+            p.ldc = a.ldc ? a.ldc : a.N;
+            p.trans_a = a.trans_a;
+            p.trans_b = a.trans_b;
+            p.A = a.A; p.B = a.B;
+            if (vnpu::k::skinny_f32_takes(p)) vnpu::k::skinny_f32_route(p, out, size);
+            else
+                std::snprintf(out, size, "%s", a.M <= 8 && !a.trans_a && !a.trans_b && vnpu::k::gemv_f32_supported(p)
+                                                   ? "gemv" : "gemm");
+            return VNPU_OK;
+        }
         if (cmd->opcode == VNPU_OP_MATMUL_I8) {   // dense weights
             const vnpu_matmul_i8_args_t &a = cmd->args.matmul_i8;
             if (!a.M || !a.N || !a.K) return VNPU_ERR_INVALID_ARGUMENT;

@@ -1343,7 +1343,6 @@ void cull_classify(hipStream_t s, const uint8_t *mask, uint32_t mask_m, uint32_t
 // state is read by the single-pass kernel).
 // A requested K depth (device tiles 128 x depth x 128) is honoured up to a
 // split-K workspace of kMaxSplitWs bytes; deeper slices beyond that.
-constexpr uint64_t kMaxSplitWs = 256ull << 20;
 
 static uint32_t gemm_f32_splits(const F32Gemm &p)
 {

@@ -148,6 +148,10 @@ void gemv_f32(hipStream_t s, const F32Gemm &p, float *ws);
 bool skinny_f32_takes(const F32Gemm &p);
 size_t skinny_f32_ws_bytes(const F32Gemm &p);
 void skinny_f32(hipStream_t s, const F32Gemm &p, float *ws);
+// Its kernel, ranges of K and estimated time, by name.
+void skinny_f32_route(const F32Gemm &p, char *out, size_t size);
+// Partial sums of K ranges take this much workspace at most.
+constexpr uint64_t kMaxSplitWs = 256ull << 20;
 // C = epilogue of the sum over z of ws[z][m][n], z ascending (gemm_f32.hip).
 void splitk_reduce(hipStream_t s, const F32Gemm &p, const float *ws, uint32_t splits);
 

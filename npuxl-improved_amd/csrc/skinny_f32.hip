@@ -26,6 +26,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cstdio>
 #include <type_traits>
 
 namespace vnpu {
@@ -195,6 +196,7 @@ struct Plan {
     enum Kind { kNone, kMatrix, kLanes } kind = kNone;   // not here, skinny_f32_kernel, gemv_f32_nt_kernel
     int cb = 4;
     uint32_t splits = 1, k_per = 0;
+    double us = 0.0;   // estimated
 };
 
 template <int MG, int CB, bool NT, int W, int U>
@@ -391,6 +393,12 @@ void launch_nt(hipStream_t s, const F32Gemm &p)
 
 namespace {
 
+// Partial sums written and read again: bytes that the second launch's 3.5 us cover
+// (481 x 3808 x 1042, 32 MB in eight ranges 65 us, 16 MB in four 70.5), and those per
+// microsecond beyond (988 x 3378 x 7616 in two ranges, 120 MB, 572 us, in one 534;
+// 382 x 1535 x 14208 217 against 197).
+constexpr double kPartialsFree = 40e6, kPartials = 2.2e6;
+
 // Microseconds of the matrix-core kernel with 16 x.cb columns a workgroup, K in
 // the number of ranges that ends first.  A workgroup alone on a CU takes 2 and
 // its bytes at `cu` or its products at 0.2, 0.28 or 0.44e6 flops (wider ones
@@ -404,14 +412,15 @@ double split(const F32Gemm &p, double cu, double mem, Plan &x)
     const uint32_t cols = 16 * x.cb, mg = p.M <= 16 ? 1 : p.M <= 32 ? 2 : 4, cus = cu_count();
     const uint64_t tiles = static_cast<uint64_t>((p.N + cols - 1) / cols) * ((p.M + 16 * mg - 1) / (16 * mg));
     double best = 0.0;
-    for (uint32_t s = 1; s == 1 || (s <= 16 && p.K / s >= 240); s *= 2) {
+    const uint64_t out_bytes = 4ull * p.M * p.N;
+    for (uint32_t s = 1; s == 1 || (s <= 16 && p.K / s >= 240 && s * out_bytes <= kMaxSplitWs); s *= 2) {
         const uint32_t k_per = ((p.K + s - 1) / s + 63) / 64 * 64;   // whole chunks
         const double bytes = 4.0 * k_per * cols, flops = 32.0 * mg * k_per * cols;
         const double alone = 2.0 + std::max(bytes / cu, flops / (x.cb == 1 ? 0.2e6 : x.cb == 2 ? 0.28e6 : 0.44e6));
         const uint64_t wgs = tiles * s;
         double t = static_cast<double>(wgs / cus) * std::max(alone, cus * bytes / mem);
         if (wgs % cus) t += std::max(alone, static_cast<double>(wgs % cus) * bytes / mem);
-        if (s > 1) t += 3.5;
+        if (s > 1) t += 3.5 + std::max(0.0, 2.0 * s * out_bytes - kPartialsFree) / kPartials;
         if (s == 1 || t < best) {
             best = t;
             x.k_per = k_per;
@@ -489,6 +498,7 @@ Plan plan(const F32Gemm &p)
         if (i == most || t < best) {
             best = t;
             x = y;
+            x.us = t;
         }
     }
     return x;
@@ -497,6 +507,14 @@ Plan plan(const F32Gemm &p)
 }  // namespace
 
 bool skinny_f32_takes(const F32Gemm &p) { return plan(p).kind != Plan::kNone; }
+
+void skinny_f32_route(const F32Gemm &p, char *out, size_t size)
+{
+    const Plan x = plan(p);
+    const int mg = p.M <= 16 ? 1 : p.M <= 32 ? 2 : 4;
+    if (x.kind == Plan::kLanes) std::snprintf(out, size, "lanes<%u>", p.M);
+    else std::snprintf(out, size, "skinny<%d,%d,%s> splits=%u us=%.1f", mg, x.cb, p.trans_b ? "NK" : "KN", x.splits, x.us);
+}
 
 size_t skinny_f32_ws_bytes(const F32Gemm &p)
 {

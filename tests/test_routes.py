@@ -99,3 +99,18 @@ def test_matmul_i8_direct_instances():
     want.remove("direct<1,1,16,stream>")
     want |= {f"direct<{i}{o}>" for i in ("2,4,4", "4,4,4") for o in ("", ",spread", ",stream")}
     assert seen == want
+
+
+def matmul_f32(M, K, N, tb=0):
+    return route(abi.OP_MATMUL_F32, A=4096, B=4096, C=4096, M=M, K=K, N=N, trans_b=tb)
+
+
+@pytest.mark.parametrize("M,K,N,tb,splits", [
+    # ranges of K against the partial sums that they write and read, us
+    (988, 3378, 7616, 0, 1),     # 120 MB in two ranges: 534 / 572
+    (382, 1535, 14208, 0, 1),    # 87 MB: 197 / 217
+    (670, 939, 1935, 1, 2),      # 21 MB: 65 / 60
+    (481, 3808, 1042, 0, 8),     # 32 MB in eight, 16 in four: 70 / 65
+    (16, 4096, 4096, 0, 4), (77, 1000, 1001, 0, 4)])
+def test_matmul_f32_ranges(M, K, N, tb, splits):
+    assert f" splits={splits} " in matmul_f32(M, K, N, tb)
