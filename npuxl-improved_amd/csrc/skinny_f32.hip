@@ -196,7 +196,6 @@ struct Plan {
     enum Kind { kNone, kMatrix, kLanes } kind = kNone;   // not here, skinny_f32_kernel, gemv_f32_nt_kernel
     int cb = 4;
     uint32_t splits = 1, k_per = 0;
-    double us = 0.0;   // estimated
 };
 
 template <int MG, int CB, bool NT, int W, int U>
@@ -214,11 +213,35 @@ void launch(hipStream_t s, const F32Gemm &p, const Plan &x, float *ws)
     skinny_f32_kernel<MG, CB, NT, W, U><<<grid, 64 * W, lds, s>>>(p, x.k_per, x.splits > 1 ? ws : nullptr);
 }
 
-// Sixteen waves a workgroup where their registers allow it (128 a lane), and
-// as many depths in flight as eight waves' 256 hold.
+// Waves of a 64 x 64 workgroup.  A wave takes 32 depths at a time: over a short K
+// most of eight have nothing to multiply, but hold LDS that another workgroup of
+// the same CU could have, and their zeros are added.  Two to K = 64, four to 128,
+// where the workgroups are more than the CUs (us with eight, four, two: 932 x 32 x
+// 9408 46, 34, 30; 700 x 32 x 2000 11.4, 8.4, 10.4; 300 x 96 x 10000 24, 20, 18).
+// Eight where they are not (512 x 100 x 1243 8.0 against 9.1 with four) and beyond
+// (290 x 202 x 7636 24.9 against 28.0).
+int waves_64x64(const F32Gemm &p, const Plan &x)
+{
+    const uint64_t wgs = static_cast<uint64_t>((p.N + 63) / 64) * ((p.M + 63) / 64) * x.splits;
+    if (x.k_per > 128 || wgs <= cu_count()) return 8;
+    return x.k_per <= 64 && wgs > 2ull * cu_count() ? 2 : 4;
+}
+
+// Otherwise sixteen waves a workgroup where their registers allow it (128 a lane),
+// and as many depths in flight as eight waves' 256 hold.
+int waves(const F32Gemm &p, const Plan &x)
+{
+    return x.cb == 4 && p.M > 32 ? waves_64x64(p, x) : x.cb == 1 && p.M <= 32 ? 16 : 8;
+}
+
 template <int MG, bool NT>
 void launch_matrix(hipStream_t s, const F32Gemm &p, const Plan &x, float *ws)
 {
+    const int w = waves(p, x);
+    if constexpr (MG == 4) {
+        if (x.cb == 4 && w == 2) return launch<MG, 4, NT, 2, 2>(s, p, x, ws);
+        if (x.cb == 4 && w == 4) return launch<MG, 4, NT, 4, 2>(s, p, x, ws);
+    }
     if (x.cb == 4) launch<MG, 4, NT, 8, 2>(s, p, x, ws);
     else if (x.cb == 2) launch<MG, 2, NT, 8, 4>(s, p, x, ws);
     else launch<MG, 1, NT, MG <= 2 ? 16 : 8, 4>(s, p, x, ws);
@@ -498,7 +521,6 @@ Plan plan(const F32Gemm &p)
         if (i == most || t < best) {
             best = t;
             x = y;
-            x.us = t;
         }
     }
     return x;
@@ -513,7 +535,8 @@ void skinny_f32_route(const F32Gemm &p, char *out, size_t size)
     const Plan x = plan(p);
     const int mg = p.M <= 16 ? 1 : p.M <= 32 ? 2 : 4;
     if (x.kind == Plan::kLanes) std::snprintf(out, size, "lanes<%u>", p.M);
-    else std::snprintf(out, size, "skinny<%d,%d,%s> splits=%u us=%.1f", mg, x.cb, p.trans_b ? "NK" : "KN", x.splits, x.us);
+    else
+        std::snprintf(out, size, "skinny<%d,%d,%s,%d> splits=%u", mg, x.cb, p.trans_b ? "NK" : "KN", waves(p, x), x.splits);
 }
 
 size_t skinny_f32_ws_bytes(const F32Gemm &p)

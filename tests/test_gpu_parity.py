@@ -657,7 +657,10 @@ def test_matmul_f32_strided_operands(gpu, M, K, N, ta, tb):
     (2, 513, 1000, 0, 0, 0), (32, 15, 7, 0, 0, 0),
     # unaligned rows with lanes along K (a last vector that K ends in), and more than 64 rows
     (2, 8193, 1026, 1, 0, 0), (8, 8450, 1001, 1, 1, 3), (77, 1003, 1001, 0, 0, 0), (130, 514, 67, 1, 0, 1),
-    (700, 513, 129, 0, 1, 0), (66, 1024, 512, 0, 0, 0), (1100, 515, 300, 0, 2, 1), (3, 3, 2, 0, 0, 0)])
+    (700, 513, 129, 0, 1, 0), (66, 1024, 512, 0, 0, 0), (1100, 515, 300, 0, 2, 1), (3, 3, 2, 0, 0, 0),
+    # 64 x 64 workgroups of two and of four waves: a depth below and past a wave's 32, past all waves'
+    (141, 31, 11523, 0, 0, 0), (139, 64, 13038, 1, 0, 0), (300, 33, 10001, 0, 1, 2), (333, 61, 9001, 1, 0, 1),
+    (72, 37, 9295, 0, 0, 0), (700, 125, 2001, 0, 0, 3), (90, 128, 9000, 1, 0, 0), (500, 99, 2500, 1, 1, 0)])
 def test_matmul_f32_few_rows(gpu, M, K, N, tb, lda_pad, ldb_pad):
     """Few rows (skinny_f32.hip) at the edges of its tiles and rules.  Every
     product and sum is f32, in chains of at most K / 16 terms: the error is

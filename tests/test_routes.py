@@ -113,4 +113,16 @@ def matmul_f32(M, K, N, tb=0):
     (481, 3808, 1042, 0, 8),     # 32 MB in eight, 16 in four: 70 / 65
     (16, 4096, 4096, 0, 4), (77, 1000, 1001, 0, 4)])
 def test_matmul_f32_ranges(M, K, N, tb, splits):
-    assert f" splits={splits} " in matmul_f32(M, K, N, tb)
+    assert matmul_f32(M, K, N, tb).endswith(f" splits={splits}")
+
+
+@pytest.mark.parametrize("M,K,N,tb,waves", [
+    # 64 x 64 workgroups over a short K, us with the waves here / with eight
+    (932, 32, 9408, 1, 2),       # 30 / 46
+    (427, 64, 13952, 0, 2),      # 26 / 34
+    (700, 32, 2000, 0, 4),       # 8.4 / 11.4
+    (796, 128, 7584, 0, 4),      # 37 / 44
+    (512, 100, 1243, 0, 8),      # with four 9.1 / 8.0
+    (290, 202, 7636, 1, 8)])     # with four 28.0 / 24.9
+def test_matmul_f32_waves(M, K, N, tb, waves):
+    assert re.fullmatch(rf"skinny<4,4,..,{waves}> splits=1", matmul_f32(M, K, N, tb))
