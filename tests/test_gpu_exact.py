@@ -169,7 +169,7 @@ def test_row_chain_add_norm_quant_bit_exact(gpu):
     (8, 32, 1, 4096, 128, 1, None),        # config-4 decode
     (1, 4, 256, 256, 128, 1, None),        # prefill tiles
     (1, 2, 300, 700, 64, 1, "inf"), (2, 2, 3, 500, 128, 0, "normal"), (1, 2, 17, 40, 64, 1, "row"),
-    (1, 2, 37, 70, 20, 0, "normal"),       # other head sizes: the row-wise kernel
+    (1, 2, 37, 70, 20, 0, "normal"),       # no multiple of 8: the row-wise kernel
     (1, 2, 9, 40, 13, 1, None), (2, 2, 3, 50, 23, 0, None), (1, 2, 6, 30, 6, 1, None),
     (1, 1, 5, 64, 96, 1, None), (2, 3, 1, 1, 128, 0, None)])
 def test_attention_reference_order_bit_exact(exact_gpu, b, h, sq, sk, d, causal, mask):

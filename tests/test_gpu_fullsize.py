@@ -255,7 +255,8 @@ def test_config5_mtp_head_softmax_full(gpu):
 
 @pytest.mark.parametrize("b,h,sq,sk,d,causal", [
     (1, 2, 1, 100, 128, 0), (2, 3, 1, 5000, 128, 1), (1, 2, 4, 3000, 64, 0), (2, 2, 2, 40, 32, 1),
-    (1, 2, 64, 200, 128, 1), (1, 2, 150, 700, 64, 0), (1, 2, 20, 50, 80, 0), (1, 1, 1, 1, 128, 0)])
+    (1, 2, 64, 200, 128, 1), (1, 2, 150, 700, 64, 0), (1, 2, 20, 50, 80, 0), (1, 1, 1, 1, 128, 0),
+    (1, 2, 20, 50, 160, 0), (1, 2, 20, 1500, 36, 1)])
 @pytest.mark.parametrize("dev", ["gpu", "fast_gpu"])
 def test_attention_neg_inf_mask(request, dev, b, h, sq, sk, d, causal):
     """Additive masks holding -inf (padding): leading keys masked, scattered

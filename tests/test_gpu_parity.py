@@ -513,11 +513,16 @@ def test_matmul_i8_register_epilogue_padded_c(gpu, tiles, epi):
 
 
 @pytest.mark.parametrize("tiles,K,M", [((256, 64, 128), 448, 320), ((128, 128, 64), 448, 320),
-                                        ((256, 64, 128), 576, 64), ((128, 128, 64), 1000, 257)])
+                                        ((256, 64, 128), 576, 64), ((128, 128, 64), 1000, 257),
+                                        # the generic kernel, asked for and as what a kernel that cannot take the rows
+                                        # leaves: a depth that is no multiple of 64, rows from any byte
+                                        ((128, 64, 128), 1000, 257), ((128, 64, 128), 448, 320),
+                                        ((256, 128, 128), 1001, 130), ((256, 64, 128), 77, 65)])
 @pytest.mark.parametrize("epi", [abi.EPI_NONE, abi.EPI_RELU, abi.EPI_SILU, abi.EPI_GELU_TANH])
 def test_matmul_i8_staged_epilogue_padded_c(gpu, tiles, K, M, epi):
     """The 64-deep pipelined kernel and the generic one store C from an LDS-
-    staged tile (row scales, column scales, bias, epilogue): with a padded C
+    staged tile (row scales, column scales, bias, epilogue), and the direct one,
+    the automatic choice, from its sums in LDS: with a padded C
     and sentinel rows after row M the padding and those rows keep their
     contents, and the values follow store_i8_c's order
     (src/kernels/kernels.cpp:526-535)."""
@@ -618,11 +623,16 @@ def test_matmul_f32_split_bf16(gpu, M, K, N, ta, tb, epi, beta):
 
 
 @pytest.mark.parametrize("M,K,N,ta,tb", [(1100, 520, 6600, 0, 0), (1300, 520, 6200, 0, 1),
-                                         (1100, 520, 1920, 1, 0), (512, 512, 512, 0, 1)])
+                                         (1100, 520, 1920, 1, 0), (512, 520, 2200, 0, 1), (512, 520, 2200, 0, 0),
+                                         (512, 512, 512, 0, 1)])
 def test_matmul_f32_strided_operands(gpu, M, K, N, ta, tb):
     """A and B with row strides above their widths on the split-bf16 paths:
     the warp-specialised kernel (B as K x N and as N x K), the four-wave tile
-    with op(A) = A^T, and a K-split small grid; to the f32 bar."""
+    with op(A) = A^T, and a K-split small grid; and on the few-rows kernel, which
+    takes the smallest; to the f32 bar."""
+    kernel = route(abi.OP_MATMUL_F32, A=4096, B=4096, C=4096, M=M, K=K, N=N, trans_a=ta, trans_b=tb,
+                   lda=(M if ta else K) + 12, ldb=(K if tb else N) + 20)
+    assert kernel.startswith("skinny" if N == 512 else "gemm")
     rng = np.random.default_rng(M + K + N + 10 * ta + tb)
     a_rows, a_cols = (K, M) if ta else (M, K)
     b_rows, b_cols = (N, K) if tb else (K, N)
@@ -644,7 +654,7 @@ def test_matmul_f32_strided_operands(gpu, M, K, N, ta, tb):
     assert rel(got, want) <= 1e-4
 
 
-@pytest.mark.parametrize("M,K,N,tb,lda_pad,ldb_pad", [
+FEW_ROWS_F32 = [  # M, K, N, trans_b, lda - K, padding of ldb
     # lanes along K ([N][K], M <= 8, from 8M weights): N % 4 rows left over, one
     # to sixteen waves a row group, a last block of 256 depths that is not whole,
     # activations staged in two chunks
@@ -660,11 +670,27 @@ def test_matmul_f32_strided_operands(gpu, M, K, N, ta, tb):
     (700, 513, 129, 0, 1, 0), (66, 1024, 512, 0, 0, 0), (1100, 515, 300, 0, 2, 1), (3, 3, 2, 0, 0, 0),
     # 64 x 64 workgroups of two and of four waves: a depth below and past a wave's 32, past all waves'
     (141, 31, 11523, 0, 0, 0), (139, 64, 13038, 1, 0, 0), (300, 33, 10001, 0, 1, 2), (333, 61, 9001, 1, 0, 1),
-    (72, 37, 9295, 0, 0, 0), (700, 125, 2001, 0, 0, 3), (90, 128, 9000, 1, 0, 0), (500, 99, 2500, 1, 1, 0)])
+    (72, 37, 9295, 0, 0, 0), (700, 125, 2001, 0, 0, 3), (90, 128, 9000, 1, 0, 0), (500, 99, 2500, 1, 1, 0),
+    # wide enough for 64 and 32 columns a workgroup with 1 to 64 rows and more, K % 4 and N % 16 left over, K split and not
+    (16, 2051, 2061, 0, 0, 0), (31, 2050, 2067, 0, 0, 0), (64, 4099, 1030, 0, 0, 0), (130, 2051, 2061, 0, 0, 0),
+    (16, 513, 8209, 1, 0, 0), (31, 2051, 2061, 1, 0, 0), (64, 2049, 2051, 1, 0, 0), (8, 35, 8507, 0, 0, 0),
+    (21, 38, 8203, 0, 0, 1), (34, 37, 9669, 0, 0, 0), (82, 35, 5277, 0, 0, 0), (5, 3943, 513, 1, 1, 0),
+    (19, 39, 10177, 1, 0, 0), (34, 37, 9066, 1, 0, 0), (76, 37, 4359, 1, 0, 0), (70, 1011, 1137, 1, 0, 3),
+    (5, 1921, 746, 1, 0, 0), (7, 4086, 277, 0, 0, 0), (4, 37, 4285, 1, 0, 0), (3, 35, 4577, 0, 0, 0),
+    (18, 41, 4197, 0, 0, 0), (18, 2111, 521, 0, 0, 0), (19, 37, 4463, 1, 0, 0), (19, 3891, 290, 1, 0, 0),
+    (43, 35, 4277, 0, 0, 0), (34, 2007, 529, 0, 0, 0), (35, 35, 4519, 1, 0, 0), (34, 2385, 519, 1, 0, 0),
+    (17, 1171, 5, 0, 0, 0), (17, 1195, 5, 1, 0, 0), (18, 39, 5, 0, 0, 0), (20, 39, 5, 1, 0, 0), (33, 765, 5, 1, 0, 0),
+    (33, 35, 5, 0, 0, 0),
+    (2, 1595, 5, 0, 0, 0), (2, 2077, 5, 1, 0, 0), (2, 8191, 1030, 1, 0, 1), (4, 8190, 1031, 1, 0, 0),
+    (6, 2917, 3053, 1, 0, 0), (7, 1331, 6505, 1, 0, 0)]
+
+
+@pytest.mark.parametrize("M,K,N,tb,lda_pad,ldb_pad", FEW_ROWS_F32)
 def test_matmul_f32_few_rows(gpu, M, K, N, tb, lda_pad, ldb_pad):
     """Few rows (skinny_f32.hip) at the edges of its tiles and rules.  Every
-    product and sum is f32, in chains of at most K / 16 terms: the error is
-    near sqrt(K / 16) 2^-24 of the largest term, below 1e-5 of the result."""
+    product and sum is f32, in chains of at most K / 2 terms (K <= 64), K / 4 (K <= 128)
+    or K / 8: the error is near sqrt(K / 8) 2^-24 of the largest term, below 1e-5 of
+    the result at any K here."""
     rng = np.random.default_rng(M + 7 * K + 13 * N)
     lda, ldb = K + lda_pad, (K if tb else N) + ldb_pad
     A = rng.standard_normal((M, lda)).astype(np.float32)
@@ -881,7 +907,9 @@ def test_rope_positions_and_identity(gpu):
     # prefill kernel (f32 MFMA, head_dim 64/128): ragged lengths, masks, offsets
     (2, 3, 129, 200, 64, 0, True), (1, 2, 256, 256, 128, 1, True), (1, 2, 100, 1000, 128, 1, False),
     (1, 1, 5, 5, 128, 1, False), (1, 2, 300, 120, 64, 1, False), (1, 1, 640, 640, 128, 1, False),
-    (1, 1, 17, 9, 64, 1, False), (1, 2, 40, 40, 80, 0, False)])
+    (1, 1, 17, 9, 64, 1, False), (1, 2, 40, 40, 80, 0, False),
+    # generic kernel on a high-throughput device, row-wise on the other
+    (1, 2, 40, 40, 160, 0, False), (1, 2, 33, 700, 36, 1, True)])
 @pytest.mark.parametrize("dev", ["gpu", "fast_gpu"])
 def test_attention(request, dev, b, h, sq, sk, d, causal, use_mask):
     """Both device modes: the default (reference order) and high throughput

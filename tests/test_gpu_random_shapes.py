@@ -58,8 +58,8 @@ def test_random_matmul_i8_pairs_small_m(gpu):
 def test_random_attention_both_devices(gpu, fast_gpu):
     """Seeded random ATTENTION_F32 calls (reference src/kernels/llm.cpp:442-546):
     batch, heads, query and key lengths (decode and prefill paths, ragged
-    64-key blocks and 128-row tiles), head sizes 64 and 128 (the tiled
-    kernels) and others (the row-wise kernel), causal offsets, additive masks
+    64-key blocks and 128-row tiles), head sizes 64 and 128, which fill a tile of
+    the reference-order kernels, and 32 and 80, causal offsets, additive masks
     with -inf runs, explicit and default scales.  The default device must give
     the reference's bits (the oracle's AVX2-order restatement); the
     high-throughput device must be within the attention bar."""

@@ -7,7 +7,7 @@ import re
 import pytest
 
 from gpu_ops import route
-from test_gpu_parity import DIRECT_I8
+from test_gpu_parity import DIRECT_I8, FEW_ROWS_F32
 from vnpu_mi355x import abi
 
 
@@ -126,3 +126,23 @@ def test_matmul_f32_ranges(M, K, N, tb, splits):
     (290, 202, 7636, 1, 8)])     # with four 28.0 / 24.9
 def test_matmul_f32_waves(M, K, N, tb, waves):
     assert re.fullmatch(rf"skinny<4,4,..,{waves}> splits=1", matmul_f32(M, K, N, tb))
+
+
+def test_matmul_f32_few_rows_instances():
+    """The few-rows kernels' GPU test runs every instance that is built, with K whole and (where it can be) in ranges."""
+    seen = set()
+    for M, K, N, tb, pad_a, pad_b in FEW_ROWS_F32:
+        t = route(abi.OP_MATMUL_F32, A=4096, B=4096, C=4096, M=M, K=K, N=N, trans_b=tb, lda=K + pad_a,
+                  ldb=(K if tb else N) + pad_b)
+        if t.startswith("skinny"):
+            seen.add((t.split()[0], not t.endswith("splits=1")))
+        else:
+            seen.add(t)
+    want = {f"lanes<{m}>" for m in range(1, 9)}
+    for b in ("KN", "NK"):
+        for mg in (1, 2, 4):
+            for cb in (1, 2, 4):
+                name = f"skinny<{mg},{cb},{b},{16 if cb == 1 and mg < 4 else 8}>"
+                want |= {(name, False), (name, True)}
+        want |= {(f"skinny<4,4,{b},{w}>", False) for w in (2, 4)}
+    assert not want - seen, sorted(map(str, want - seen))
