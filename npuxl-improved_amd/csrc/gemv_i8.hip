@@ -24,9 +24,8 @@
 //   * the activations (M x K int8, tiny) are staged in LDS as [k/16][m][16]
 //     (dynamic LDS sized to the chunk actually used), so lane kg reads its
 //     16 bytes of every row with one ds_read_b128 per row; the matrix-core
-//     kernel instead reads them from global memory with
-//     each weight block when the rows are 16-byte aligned
-//     (gemv_i8_mfma_direct);
+//     kernel reads them from global memory with each weight block when the
+//     rows are 16-byte aligned (gemv_i8_mfma_direct);
 //   * v_dot4_i32_i8 (4 per 16 bytes per row) accumulates in int32 for up
 //     to four rows; from five rows one v_mfma_i32_16x16x64_i8 per block
 //     does it (gemv_i8_mfma below);
@@ -245,7 +244,7 @@ __global__ __launch_bounds__(64 * W) void gemv_i8_mfma(I8GemmPair ps, uint32_t g
     const bool second = blockIdx.x >= grid0;
     const I8Gemm &p = ps.p[second ? 1 : 0];
     const uint32_t bx = second ? blockIdx.x - grid0 : blockIdx.x;
-    static_assert(M <= 16, "one 16-row group");
+    static_assert(M <= kGemvMaxRows, "the rows of one 16-row group");
     typedef int v4i __attribute__((ext_vector_type(4)));
     extern __shared__ __attribute__((aligned(16))) int8_t a_lds[];  // [chunk_k/16][M][16]
     __shared__ int red[W][T][M][16];
@@ -351,7 +350,7 @@ __global__ __launch_bounds__(64 * W) void gemv_i8_mfma(I8GemmPair ps, uint32_t g
 template <int M, int W, int U, int T>
 __global__ __launch_bounds__(64 * W) void gemv_i8_mfma_direct(I8GemmPair ps, uint32_t grid0)
 {
-    static_assert(M <= 16, "one 16-row group");
+    static_assert(M <= kGemvMaxRows, "the rows of one 16-row group");
     const bool second = blockIdx.x >= grid0;
     const I8Gemm &p = ps.p[second ? 1 : 0];
     const uint32_t nt0 = (second ? blockIdx.x - grid0 : blockIdx.x) * T;
@@ -375,8 +374,8 @@ __global__ __launch_bounds__(64 * W) void gemv_i8_mfma_direct(I8GemmPair ps, uin
         rw[t] = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(strip) + static_cast<uint64_t>(first) * 1024,
                                                   0, bytes, kBufferWord3);
     }
-    // A: one buffer over the Mr rows; the lane's offset is past the end for a
-    // row past Mr, a block past the wave's last or k past K
+    // A: one buffer over the M rows; the lane's offset is past the end for a
+    // row past M, a block past the wave's last or k past K
     const auto ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(p.A), 0,
                                                       static_cast<int>((M - 1) * p.lda + p.K), kBufferWord3);
     const bool row_live = row < M;

@@ -143,8 +143,9 @@ void gemm_f32(hipStream_t s, const F32Gemm &p, float *ws);
 size_t gemv_f32_ws_bytes(const F32Gemm &p);
 bool gemv_f32_supported(const F32Gemm &p);
 void gemv_f32(hipStream_t s, const F32Gemm &p, float *ws);
-// Few rows (skinny_f32.hip): M <= 64, op(A) = A, no cull and no requested K
-// depth, where it is the faster one; ws holds skinny_f32_ws_bytes(p).
+// Few rows, small weights and unaligned rows (skinny_f32.hip): M <= 2048, op(A) =
+// A, no cull, no requested K depth and rows below 2^22 floats, where it is the
+// faster one; ws holds skinny_f32_ws_bytes(p).
 bool skinny_f32_takes(const F32Gemm &p);
 size_t skinny_f32_ws_bytes(const F32Gemm &p);
 void skinny_f32(hipStream_t s, const F32Gemm &p, float *ws);

@@ -1,5 +1,6 @@
-// skinny_f32.hip - MATMUL_F32 and MTP_HEAD_F32 with few rows (M <= 64): one
-// read of B at the memory's rate.
+// skinny_f32.hip - MATMUL_F32 and MTP_HEAD_F32 with few rows: one read of B at
+// the memory's rate; and, up to 2048 rows, small weights and rows that are not
+// 16-byte aligned (the rules are at plan()).
 //
 // Replaces the reference's f32 decode kernels (src/kernels/kernels.cpp:454-520)
 // and, for an output head, execute_mtp_head (src/core/scheduler.cpp:610-641).
@@ -427,7 +428,7 @@ constexpr double kPartialsFree = 40e6, kPartials = 2.2e6;
 // its bytes at `cu` or its products at 0.2, 0.28 or 0.44e6 flops (wider ones
 // reuse more); a round of one per CU takes no less than its bytes at `mem`
 // (bytes per microsecond, measured on this kernel's reads); ranges cost the
-// second launch that adds them (3.5).  [K][N]
+// second launch that adds them (3.5) and their partial sums.  [K][N]
 // N = K = 4096 at one range 28, two 19.2, four 15.5, eight 15.6; K = 11008 N =
 // 4096 70, 42, 31.9, 32.3; K = 4096 N = 20000 64, 56, 51.7.
 double split(const F32Gemm &p, double cu, double mem, Plan &x)
@@ -461,25 +462,29 @@ double split(const F32Gemm &p, double cu, double mem, Plan &x)
 //     matrix-core kernel starts faster (8 x 1024 x 4096 14 -> 6.1 against 8.3
 //     with lanes along K).
 //   [N][K] M <= 32: 16 x 4096 x 4096 36 -> 22, x 32000 184 -> 145; 32 x 8192 x
-//     8192 101 -> 86, but x 11008 x 4096 71 against 75.  Aligned M <= 64 only up to 8M weights: 64 x 2048 x 2048
-//     18.5 -> 15, but x 4096 x 11008 81 against 93.
+//     8192 101 -> 86, but x 11008 x 4096 71 against 75.  Aligned M <= 64 only up to
+//     8M weights: 64 x 2048 x 2048 18.5 -> 15, but x 4096 x 11008 81 against 93.
 //   [K][N] M <= 4: up to N = 4096 or 8M weights (4 x 4096 x 4096 19.8 -> 15.6,
 //     x 1024 x 1024 13 -> 6); wider, or with unaligned rows from 2M weights, the
 //     split kernel's 1 KiB rows are as fast or faster (1 x 4096 x 11008 31
 //     against 35, 1 x 4096 x 4095 16.5 against 20).
 //   [K][N] M <= 8: up to N = 20480 (8 x 4096 x 16384 55 -> 42); wider, the wide
-//     kernel (8 x 4096 x 32000 84 against 87).
+//     kernel (8 x 4096 x 32000 84 against 87).  That one starts at 25600 even
+//     columns: between the two, and at odd widths, gemv_f32_kernel runs, as it did
+//     (1 x 1071 x 21049 21 against 25, but 6 x 212 x 21456 15 against 6.5).
 //   [K][N] M <= 64: 16 x 4096 x 4096 39 -> 16.5, 32 x 4096 x 32000 195 -> 105,
 //     64 x 8192 x 8192 109 -> 82.
 //   Aligned M > 64 only while the weights are so few that tiles of 128 leave the
 //     chip idle: 400 x 512 x 512 15 -> 8, 128 x 1024 x 1024 15 -> 10, 128 x 1024 x
 //     4096 24 -> 19; but 256 x 4096 x 1024 26 against 27, 200 x 2048 x 2048 24
-//     against 27.
+//     against 27.  Over a short K and wide outputs those tiles are faster still
+//     (796 x 128 x 7584 14 against 37, 932 x 32 x 9408 16 against 30), with ten times
+//     the error (4.4e-6 against 1e-7): such calls stay in full f32.
 //   Unaligned rows ran on the fp32 tile kernel from M = 9 on: 16 x 4096 x 4095
 //     70 -> 21, 128 x 4095 x 4096 90 -> 47, 700 x 4095 x 4096 577 -> 228, 2000 x
 //     1000 x 1001 154 -> 48.  Its 128-row tiles win back many rows over a short K
 //     or, [N][K], wide weights (2048 x 333 x 4000 93 against 96; [N][K] 1000 x
-//     2047 x 11007 684 against 777).
+//     2047 x 11007 684 against 777); up to 15% on either side of these lines.
 Plan plan(const F32Gemm &p)
 {
     Plan x;
