@@ -1046,8 +1046,8 @@ double general_us(const Attn &a)
 // 8 x 32 heads of 80 over 4096 keys 596 -> 138; but few rows or heads behind a
 // long context are a chain of blocks there and split over keys in attn_kernel (8
 // heads of 8, 21 rows, 1986 keys 105 against 27 us; 2 of 112, 21 rows, 2294 keys
-// 166 against 66).  Of the 996 calls of the fit the slower one is taken for five
-// by more than 5% (with the reference-order kernels for all, for 112).
+// 166 against 66).  Of 2312 calls the slower one is taken for 13 by more than 5%
+// (with the reference-order kernels for all, for one in nine).
 bool use_exact_tiled(const Attn &a)
 {
     if (use_rowwise(a)) return false;

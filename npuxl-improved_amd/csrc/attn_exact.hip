@@ -1119,9 +1119,11 @@ bool attention_exact_decodes(const Attn &a)
 double attention_exact_us(const Attn &a)
 {
     if (attention_exact_decodes(a)) return decode_us(a);
-    // share_rows' estimates, 4.1 and 11.5 us a block at head_dim 128
-    const double tiles = (a.head_dim <= 64 ? 3.05 : 4.0) * std::min(grid_blocks(a, XQW, 1.2), 2.8 * grid_blocks(a, XQ, 0.45));
-    return a.seq_q <= kDecMaxRows ? std::max(tiles, few_rows_us(a)) : tiles;
+    // share_rows' estimates, 4.1 and 11.5 us a block at head_dim 128; a mask's loads
+    // stand in each block's way (64 heads of 48, 21 rows, 1500 keys 109 us)
+    double t = (a.head_dim <= 64 ? 3.05 : 4.0) * std::min(grid_blocks(a, XQW, 1.2), 2.8 * grid_blocks(a, XQ, 0.45));
+    if (a.seq_q <= kDecMaxRows) t = std::max(t, few_rows_us(a));
+    return a.mask ? 1.15 * t : t;
 }
 
 const char *attention_exact_route(const Attn &a)
