@@ -312,12 +312,13 @@ bool direct_i8_takes(const I8Gemm &p)
     if (p.K % 64 || p.lda % 16 || reinterpret_cast<uintptr_t>(p.A) % 16) return true;
     // The staged tiles, 256 x 128: 8.8 us and 4 us for 1024 depths of a round of
     // the 128-deep ones, 10.5 and 10.7 of the 64-deep ones that K % 128 = 64
-    // leaves, fitted to 96..512 rows at the sizes above and to K = 320 to 8256.
-    // The call is theirs unless the estimates differ by 10%.
+    // leaves, fitted to 96..512 rows at the sizes above and to K = 320 to 8256; the
+    // latter less for fewer rows to store, which shows over a short K (98 x 64 x 24512
+    // 7.6 us against 9.1 here).  The call is theirs unless the estimates differ by 10%.
     const uint64_t cols = (p.N + 127) / 128, tiles = cols * ((p.M + 255) / 256);
     const uint64_t rounds = (tiles + cu_count() - 1) / cu_count();
     const bool deep = p.K % 128 == 0;
-    const double staged = (deep ? 8.8 : 10.5) +
+    const double staged = (deep ? 8.8 : 7.9 + 2.6 * std::min(p.M, 256u) / 256) +
                           std::hypot(rounds * (deep ? 4.0 : 10.7) * p.K / 1024, memory_us(p, cols, 256));
     double direct;
     choose(p, direct);

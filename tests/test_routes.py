@@ -151,3 +151,15 @@ def test_matmul_f32_few_rows_instances():
                 want |= {(name, False), (name, True)}
         want |= {(f"skinny<4,4,{b},{w}>", False) for w in (2, 4)}
     assert not want - seen, sorted(map(str, want - seen))
+
+
+@pytest.mark.parametrize("M,K,N,want", [
+    # direct kernel against the 64-deep staged tiles over a short K, us
+    (98, 64, 24512, "gemm"),        # 9.1 / 7.6
+    (64, 192, 32000, "gemm"),       # 9.0 / 8.1
+    (98, 64, 8192, "direct"),       # 5.1 / 7.0
+    (64, 320, 16384, "direct"),     # 6.2 / 8.4
+    (256, 192, 8192, "direct"),     # 8.9 / 11.0
+    (256, 320, 16384, "gemm")])
+def test_matmul_i8_short_depth(M, K, N, want):
+    assert route(abi.OP_MATMUL_I8, A=4096, M=M, K=K, N=N).startswith(want)
